@@ -32,14 +32,18 @@ namespace spk {
 // The y pass of a quasi-2D grid (NZ = 2: two columns of adjacent complex values
 // per x) uses TC = 2 with one plane per block, so that every lane has a column and
 // a wave reads 32 consecutive lines' two values as one contiguous run.
-template <class T, int N, int DIR, int AXIS, int TC = strided_tcols(N)>
+// PRUNE (forward y pass of the RHS products): line point n goes to row
+// prod_row(n) and the masked rows are not stored; in place, since a tile reads
+// its whole lines before it stores and no tile touches another's columns.
+template <class T, int N, int DIR, int AXIS, int TC = strided_tcols(N), bool PRUNE = false>
 __global__ __launch_bounds__(TC * strided_tpl(N)) void k_pass_strided(
     const cpx<T> *in, cpx<T> *out, long long ncols, long long lstride, long long ostride,
     int nouter, long long fs_in, long long fs_out, const cpx<T> *__restrict__ tw, T scale,
-    const int *__restrict__ gate, Batch bt) {
+    const int *__restrict__ gate, ProdLay pl, cpx<T> *probe, Batch bt) {
     in = rebase(bt, 0, in);
     out = rebase(bt, 1, out);
     gate = rebase(bt, 2, gate);
+    if constexpr (PRUNE) probe = rebase(bt, 3, probe);
     if (gate != nullptr && *gate == 0) return;
     constexpr int E = strided_e(N);
     constexpr int TPL = N / E;
@@ -63,7 +67,16 @@ __global__ __launch_bounds__(TC * strided_tpl(N)) void k_pass_strided(
         v[i] = cscale(a, scale);
     }
     LineFFT<T, N, E, DIR>::run(v, lds + c * LL, t, tw);
-    if (active) {
+    if constexpr (PRUNE) {
+        if (active) {
+            if (t == 0 && col == 0) probe[(long long)blockIdx.y * nouter + o] = v[0];
+#pragma unroll
+            for (int i = 0; i < E; i++) {
+                const int r = prod_row(pl, t + i * TPL);
+                if (r >= 0) out[base_out + (long long)r * lstride] = v[i];
+            }
+        }
+    } else if (active) {
 #pragma unroll
         for (int i = 0; i < E; i++) out[base_out + (long long)(t + i * TPL) * lstride] = v[i];
     }
@@ -182,6 +195,9 @@ static const cpx<T> *tw_ptr(const Twiddles &tw, long long off) {
 // launchers
 // ------------------------------------------------------------------------
 
+// plain passes: no pruning
+static const ProdLay NO_PRUNE{0, 0, 0, 0, 0};
+
 #define SPK_POW2_CASES(X) X(2) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024) X(2048)
 
 template <class T, int DIR, int AXIS>
@@ -198,7 +214,7 @@ static int launch_strided(spk_ctx ctx, int n, long long ncols, long long lstride
                 dim3 grid((unsigned)nouter, a.nfields, nbz);                                      \
                 k_pass_strided<T, NN, DIR, AXIS, 2><<<grid, 2 * strided_tpl(NN), 0, ctx->stream>>>(   \
                     (const cpx<T> *)a.in, (cpx<T> *)a.out, ncols, lstride, ostride, nouter,         \
-                    a.fstride_in, a.fstride_out, twp, (T)a.scale, ctx->gate, bt);                  \
+                    a.fstride_in, a.fstride_out, twp, (T)a.scale, ctx->gate, NO_PRUNE, nullptr, bt); \
                 break;                                                                             \
             }                                                                                      \
         }                                                                                          \
@@ -206,7 +222,7 @@ static int launch_strided(spk_ctx ctx, int n, long long ncols, long long lstride
         dim3 grid((unsigned)ntiles, a.nfields, nbz);                                               \
         k_pass_strided<T, NN, DIR, AXIS, TC><<<grid, TC * strided_tpl(NN), 0, ctx->stream>>>(         \
             (const cpx<T> *)a.in, (cpx<T> *)a.out, ncols, lstride, ostride, nouter, a.fstride_in, \
-            a.fstride_out, twp, (T)a.scale, ctx->gate, bt);                                        \
+            a.fstride_out, twp, (T)a.scale, ctx->gate, NO_PRUNE, nullptr, bt);                     \
         break;                                                                                     \
     }
     switch (n) {
@@ -242,6 +258,48 @@ int launch_pass_y(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, int 
     const long long plane = (long long)g.ny * g.nzh;
     if (dir < 0) return pass_dispatch<-1, 1>(ctx, g.ny, g.nzh, g.nzh, plane, g.nx, tw, tw.off_y, tin, tout, a);
     return pass_dispatch<+1, 1>(ctx, g.ny, g.nzh, g.nzh, plane, g.nx, tw, tw.off_y, tin, tout, a);
+}
+
+template <class T>
+static int launch_y_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, void *P, int n, const ProdLay &l,
+                             void *probe) {
+    const cpx<T> *twp = tw_ptr<T>(tw, tw.off_y);
+    cpx<T> *p = (cpx<T> *)P, *pr = (cpx<T> *)probe;
+    Batch bt;
+    SPK_TRY(make_batch(ctx, {P, P, ctx->gate, probe}, &bt));
+    const unsigned nbz = nboxes(ctx);
+#define SPK_YP_CASE(NN)                                                                                     \
+    case NN: {                                                                                              \
+        constexpr int TC = strided_tcols_t<T>(NN);                                                          \
+        const long long ntiles = ((long long)l.kc * g.nx + TC - 1) / TC;                                    \
+        dim3 grid((unsigned)ntiles, n, nbz);                                                                \
+        k_pass_strided<T, NN, -1, 1, TC, true><<<grid, TC * strided_tpl(NN), 0, ctx->stream>>>(             \
+            p, p, l.kc, l.kp, l.xs, g.nx, g.ntc, g.ntc, twp, (T)1, ctx->gate, l, pr, bt);                   \
+        break;                                                                                              \
+    }
+    switch (g.ny) {
+        SPK_POW2_CASES(SPK_YP_CASE)
+        default:
+            set_error("line length %d not supported (power of two 2..2048)", g.ny);
+            return SPK_ERR_ARG;
+    }
+#undef SPK_YP_CASE
+    SPK_LAUNCH_CHECK();
+    return SPK_OK;
+}
+
+int launch_pass_y_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, void *P, int n, const ProdLay &l,
+                           void *probe) {
+    return tw.prec == SPK_F64 ? launch_y_products<double>(ctx, g, tw, P, n, l, probe)
+                              : launch_y_products<float>(ctx, g, tw, P, n, l, probe);
+}
+
+// the pad columns of a row (kc <= k < kp) are transformed with the others and
+// never read
+int launch_pass_x_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, void *P, int n, const ProdLay &l) {
+    const PassArgs a{P, P, n, g.ntc, g.ntc, 1.0};
+    return pass_dispatch<-1, 0>(ctx, g.nx, (long long)(g.ny - l.nskip) * l.kp, l.xs, 0, 1, tw, tw.off_x, tw.prec,
+                                tw.prec, a);
 }
 
 #define SPK_Z_CASES(X) X(2) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)

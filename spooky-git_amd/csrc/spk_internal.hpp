@@ -133,6 +133,13 @@ int launch_pass_x(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, int 
                   const PassArgs &a);
 int launch_pass_y(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, int tin, int tout,
                   const PassArgs &a);
+// forward y pass of n products from the z pass (first kc columns of every row)
+// into the rows the mask keeps, in place (layout l); probe[f nx + x]: mode
+// (k_y, k_z) = 0 of field f at x, which is NaN exactly when plane x holds a NaN
+int launch_pass_y_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, void *P, int n, const ProdLay &l,
+                           void *probe);
+// forward x pass of those products, in place
+int launch_pass_x_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, void *P, int n, const ProdLay &l);
 // z R2C (real padded rows -> complex rows) and C2R (complex rows -> real padded rows)
 int launch_pass_z_r2c(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int tin, int tout,
                       const PassArgs &a);
@@ -150,7 +157,7 @@ void solver_advance_host(spk_solver s, int n);
 // batch slots of a solver's arrays
 enum : int {
     SL_U = 0, SL_S, SL_DU, SL_REAL, SL_W, SL_P, SL_W2, SL_P2, SL_BREAL, SL_TS, SL_PMAX, SL_UC0, SL_UC1, SL_DU0,
-    SL_PLAN, SL_COUNT
+    SL_PLAN, SL_PROBE, SL_COUNT
 };
 static_assert(SL_COUNT <= BOX_SLOTS, "batch slots");
 // the row of s in a batch table (arrays by slot, coefficients) and the byte

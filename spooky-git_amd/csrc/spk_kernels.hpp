@@ -238,7 +238,7 @@ template <class T, int NZ, int PROG, bool BAT = false>
 __global__ __launch_bounds__(256) void k_zmid(const cpx<T> *__restrict__ W, const cpx<T> *__restrict__ Wr,
                                               cpx<T> *__restrict__ P, long long nrows, long long fs,
                                               const cpx<T> *__restrict__ tw_nz,
-                                              const cpx<T> *__restrict__ tw_m, ZConst zc,
+                                              const cpx<T> *__restrict__ tw_m, ZConst zc, ProdLay pl, int ny,
                                               double *__restrict__ pmax, const int *__restrict__ gate, Batch bt) {
     if constexpr (BAT) {
         W = rebase(bt, 0, W);
@@ -324,6 +324,9 @@ __global__ __launch_bounds__(256) void k_zmid(const cpx<T> *__restrict__ W, cons
         }
     }
 
+    // the product rows' place, and only the modes the mask keeps (ProdLay)
+    const int xp = (int)row / ny;
+    cpx<T> *dst = P + xp * pl.xs + ((int)row - xp * ny) * (long long)pl.kp;
 #pragma unroll
     for (int q = 0; q < Z::NOUT; q++) {
         cpx<T> v[E];
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(256) void k_zmid(const cpx<T> *__restrict__ W, cons
             }
             v[i] = cpx<T>{zproduct<PROG>(q, ae, zc), zproduct<PROG>(q, ao, zc)};
         }
-        Row::r2c_tw(v, active, P + q * fs + row * NZH, L, t, rt);
+        Row::r2c_tw(v, active, dst + q * fs, L, t, rt, pl.kc);
     }
 }
 
@@ -368,6 +371,7 @@ struct EpiConst {
     double nu, nu_m, nu_th, N2, shear, omega;
     int oT, oE, oQ, oA;
     double gam, xi;  // gammaRK, xiRK of the stage
+    ProdLay pl;      // layout of the products
 };
 
 __device__ __forceinline__ cpx<double> cadd(cpx<double> a, cpx<double> b) { return {a.x + b.x, a.y + b.y}; }
@@ -418,7 +422,12 @@ __global__ __launch_bounds__(256) void k_epilogue(const cpx<T> *__restrict__ P, 
         d[f] = cpx<double>{0.0, 0.0};
         u[f] = U[f * N + idx];
     }
-    auto prod = [&](int q) { return cconv<double>(P[(long long)q * N + idx]); };
+    // a mode outside the mask's columns has no product stored: it takes mode
+    // (i, 0, 0) instead, times m = 0 (NaN stays NaN: a transform of data with a
+    // NaN is NaN in every mode)
+    const int prow = k < c.pl.kc ? prod_row(c.pl, j) : -1;
+    const long long pidx = (long long)i * c.pl.xs + (prow >= 0 ? (long long)prow * c.pl.kp + k : 0);
+    auto prod = [&](int q) { return cconv<double>(P[(long long)q * N + pidx]); };
 
     // HyperbolicTerms (physics.cu:30-103)
     if constexpr (L::INC) {
@@ -565,6 +574,35 @@ struct FusedConst {
     double cu, cs;  // coefficients of the stored increment in the current state and the base
 };
 
+// Column tiles of the fused kernel: tile T holds the TC columns from T TC on of
+// the flattened (k_y, k_z) index, so that its accesses to the state and to W
+// start on whole 128-byte lines (a tile list cut at the mask's edges instead,
+// 85 of 129 columns, ran 20% slower: 1449 against 1207 us at 256^3 FP64 stage
+// 2).  A tile with no column in the mask (fx_masked_tile) transforms no
+// product; in the others a column without products reads the (k_y, k_z) = 0
+// column's and multiplies it by m = 0.
+// Tiles without products are cheaper, and they come in runs of rows: an XCD
+// takes every eighth run of 32 tiles (one per CU at a time, neighbours sharing
+// its L2), and the rows past the masked ones come first.
+__device__ __forceinline__ int fx_tile(int b, int nt, int first) {
+    const int cs = nt >= 1024 ? 32 : (nt >= 64 ? nt >> 5 : 1);
+    const int span = 8 * cs, full = nt - nt % span;
+    int tile = b;
+    if (b < full) {
+        const int w = b / span, i = b - w * span;
+        tile = w * span + (i & 7) * cs + (i >> 3);
+    }
+    tile += first;
+    return tile < nt ? tile : tile - nt;
+}
+__device__ __forceinline__ bool fx_masked_tile(const EpiConst &c, int c0, int c1) {
+    int j = c0 / c.kg.nzh;
+    if (c0 - j * c.kg.nzh < c.pl.kc && prod_row(c.pl, j) >= 0) return false;
+    for (j++; j * c.kg.nzh < c1; j++)
+        if (prod_row(c.pl, j) >= 0) return false;
+    return true;
+}
+
 // vmcnt(0) and lgkmcnt(0) waits (gfx9 s_waitcnt encodings; other counters at
 // their maxima)
 #define SPK_WAIT_VMCNT0() __builtin_amdgcn_s_waitcnt(0x0F70)
@@ -583,11 +621,14 @@ struct FusedConst {
 // stores the same values as that column's own lane, so no memory operation sits
 // behind a branch.  Element offsets inside a field fit 32 bits and are added to
 // wave-uniform field bases.
-template <class T, int N, int LY, int MODE, int EF, int GRP, bool STRAT = false>
-__device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restrict__ U, cpx<T> *__restrict__ R,
+// MASKED: a tile of columns without products (fx_masked_tile); the accumulators are
+// 0, or NaN where a product holds one (probe, written by the forward y pass).
+template <class T, int N, int LY, int MODE, int EF, int GRP, bool MASKED, bool STRAT = false>
+__device__ __forceinline__ void fx_group(const cpx<T> *P, const cpx<T> *__restrict__ probe,
+                                         cpx<double> *__restrict__ U, cpx<T> *__restrict__ R,
                                          cpx<T> *__restrict__ W, const FusedConst &fc,
                                          const cpx<T> *__restrict__ tw, cpx<T> *twl, cpx<T> *ldsc, cpx<T> *pbuf,
-                                         const TimeState *__restrict__ ts, int tid, int nt, int t, long long col) {
+                                         const TimeState *__restrict__ ts, int tid, int nt, int t, int col) {
     using L = Layout<LY>;
     constexpr int E = fx_e(N, EF);
     constexpr int TPL = N / E;
@@ -604,8 +645,12 @@ __device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restric
     const long long N0 = c.ntc;
     const unsigned ncols = (unsigned)((long long)c.kg.ny * c.kg.nzh);
     const unsigned ucol = (unsigned)col;
-    const int j = (int)(col / c.kg.nzh);
-    const int kk = (int)(col - (long long)j * c.kg.nzh);
+    const int j = col / c.kg.nzh;
+    const int kk = col - j * c.kg.nzh;
+    // the column in the products
+    const unsigned pxs = (unsigned)c.pl.xs;
+    const int prow = kk < c.pl.kc ? prod_row(c.pl, j) : -1;
+    const unsigned pcol = prow >= 0 ? (unsigned)(prow * c.pl.kp + kk) : 0u;
     const int p0 = GRP == 0 ? c.oT : (GRP == 1 ? c.oE : c.oQ);
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -627,7 +672,7 @@ __device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restric
         const cpx<T> *src = P + (long long)(p0 + q) * N0;
 #pragma unroll
         for (int i = 0; i < E; i++) {
-            const cpx<T> *g = src + (ucol + (unsigned)(t + i * TPL) * ncols);
+            const cpx<T> *g = src + (pcol + (unsigned)(t + i * TPL) * pxs);
             if constexpr (DMA)
                 __builtin_amdgcn_global_load_lds((const void *)g,
                                                  (__attribute__((address_space(3))) void *)(pbuf + (wv * E + i) * 64),
@@ -636,15 +681,31 @@ __device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restric
                 vn[i] = *g;
         }
     };
-    fetch(0);
+    if constexpr (!MASKED) fetch(0);
     // Twiddles are read from LDS: a global twiddle load would wait for every
     // earlier vector memory operation (they retire in issue order), i.e. for the
     // next product's prefetch and for the state stores.
     for (int e = tid; e < N; e += nt) twl[e] = tw[e];
-    __syncthreads();
+    if constexpr (MASKED) {
+        T s = (T)0;
+        for (int e = tid; e < N; e += nt)
+#pragma unroll
+            for (int q = 0; q < NPROD; q++) {
+                const cpx<T> a = probe[(p0 + q) * N + e];
+                s += (T)0 * a.x + (T)0 * a.y;
+            }
+        if (__syncthreads_or(!(s == (T)0))) {
+#pragma unroll
+            for (int q = 0; q < NCOMP; q++)
+#pragma unroll
+                for (int i = 0; i < E; i++) acc[q][i] = cpx<double>{__builtin_nan(""), __builtin_nan("")};
+        }
+    } else {
+        __syncthreads();
+    }
 
 #pragma unroll 1
-    for (int q = 0; q < NPROD; q++) {
+    for (int q = 0; q < (MASKED ? 0 : NPROD); q++) {
         cpx<T> v[E];
         if constexpr (DMA) {
             SPK_WAIT_VMCNT0();
@@ -827,18 +888,18 @@ __device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restric
 
 // STRAT (Boussinesq layouts with stratification): the temperature group and
 // then the velocity group in the first grid row's blocks, grid y = 1 + MHD
-template <class T, int N, int LY, int MODE, int EF, bool BAT = false, bool STRAT = false>
+template <class T, int N, int LY, int MODE, int EF, bool STRAT = false>
 __global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilogue(
-    const cpx<T> *P, cpx<double> *__restrict__ U, cpx<T> *__restrict__ S, cpx<T> *__restrict__ W,
-    FusedConst fc, const cpx<T> *__restrict__ tw, const TimeState *__restrict__ ts, Batch bt) {
+    const cpx<T> *P, const cpx<T> *__restrict__ probe, cpx<double> *__restrict__ U, cpx<T> *__restrict__ S,
+    cpx<T> *__restrict__ W, FusedConst fc, const cpx<T> *__restrict__ tw, const TimeState *__restrict__ ts, Batch bt) {
     using L = Layout<LY>;
-    if constexpr (BAT) {
-        P = rebase(bt, 0, P);
-        U = rebase(bt, 1, U);
-        S = rebase(bt, 2, S);
-        W = rebase(bt, 3, W);
-        ts = rebase(bt, 4, ts);
-        const BoxRow *br = batch_row(bt);
+    P = rebase(bt, 0, P);
+    U = rebase(bt, 1, U);
+    S = rebase(bt, 2, S);
+    W = rebase(bt, 3, W);
+    ts = rebase(bt, 4, ts);
+    probe = rebase(bt, 5, probe);
+    if (const BoxRow *br = batch_row(bt)) {
         fc.e.nu = br->nu;
         fc.e.nu_m = br->nu_m;
         fc.e.nu_th = br->nu_th;
@@ -851,33 +912,45 @@ __global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilog
     __shared__ cpx<T> lds[E != N ? TC * LL : 1];
     __shared__ cpx<T> twl[N];
     __shared__ cpx<T> pbuf[sizeof(cpx<T>) == 16 ? NT * E : 1];
-    const long long ncols = (long long)fc.e.kg.ny * fc.e.kg.nzh;
     const int tid = threadIdx.x;
-    const int cl = tid % TC, t = tid / TC;
-    long long col = (long long)xcd_remap(blockIdx.x, gridDim.x) * TC + cl;
-    if (col >= ncols) col = ncols - 1;
+    const int cl = tid % TC;
+    int t = tid / TC;
+    const int ncols = fc.e.kg.ny * fc.e.kg.nzh;
+    // the first tile past the masked rows
+    const int first = fc.e.pl.nskip > 0 ? (fc.e.pl.jc + 1 + fc.e.pl.nskip) * fc.e.kg.nzh / TC : 0;
+    const int c0 = fx_tile(blockIdx.x, gridDim.x, first) * TC;
+    const bool masked = fx_masked_tile(fc.e, c0, c0 + TC < ncols ? c0 + TC : ncols);
+    int col = c0 + cl < ncols ? c0 + cl : ncols - 1;
     cpx<T> *ldsc = lds + cl * LL;
     // group: 0 velocity (+ temperature with STRAT), then magnetic (MHD), then
     // temperature (boussinesq without STRAT)
     const int g = blockIdx.y;
-    if (g == 0) {
-        if constexpr (L::BOUSS && STRAT) {
-            fx_group<T, N, LY, MODE, EF, 2, true>(P, U, S, W, fc, tw, twl, ldsc, pbuf, ts, tid, NT, t, col);
-            // the velocity group's per-point values are computed anew, not kept
-            // live across the temperature group
-            int t2 = t;
-            long long col2 = col;
-            asm volatile("" : "+v"(t2));
-            asm volatile("" : "+v"(col2));
-            fx_group<T, N, LY, MODE, EF, 0, true>(P, U, S, W, fc, tw, twl, ldsc, pbuf, ts, tid, NT, t2, col2);
-        } else {
-            fx_group<T, N, LY, MODE, EF, 0>(P, U, S, W, fc, tw, twl, ldsc, pbuf, ts, tid, NT, t, col);
-        }
-    } else if (L::MHD && g == 1) {
-        fx_group<T, N, LY, MODE, EF, 1>(P, U, S, W, fc, tw, twl, ldsc, pbuf, ts, tid, NT, t, col);
-    } else if constexpr (L::BOUSS && !STRAT) {
-        fx_group<T, N, LY, MODE, EF, 2>(P, U, S, W, fc, tw, twl, ldsc, pbuf, ts, tid, NT, t, col);
+#define SPK_FX(GRP_, MASKED_, STRAT_) \
+    fx_group<T, N, LY, MODE, EF, GRP_, MASKED_, STRAT_>(P, probe, U, S, W, fc, tw, twl, ldsc, pbuf, ts, tid, NT, t, col)
+#define SPK_FX_GROUPS(MASKED_)                                                        \
+    if (g == 0) {                                                                     \
+        if constexpr (L::BOUSS && STRAT) {                                            \
+            SPK_FX(2, MASKED_, true);                                                 \
+            /* the velocity group's per-point values are computed anew, not kept      \
+               live across the temperature group */                                   \
+            asm volatile("" : "+v"(t));                                               \
+            asm volatile("" : "+v"(col));                                             \
+            SPK_FX(0, MASKED_, true);                                                 \
+        } else {                                                                      \
+            SPK_FX(0, MASKED_, false);                                                \
+        }                                                                             \
+    } else if (L::MHD && g == 1) {                                                    \
+        SPK_FX(1, MASKED_, false);                                                    \
+    } else if constexpr (L::BOUSS && !STRAT) {                                        \
+        SPK_FX(2, MASKED_, false);                                                    \
     }
+    if (masked) {
+        SPK_FX_GROUPS(true)
+    } else {
+        SPK_FX_GROUPS(false)
+    }
+#undef SPK_FX_GROUPS
+#undef SPK_FX
 }
 
 }  // namespace spk

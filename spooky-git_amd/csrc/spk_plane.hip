@@ -50,13 +50,15 @@ using PlaneFFT = LineFFT<T, NY, NY / PL_TPL, DIR, true, 0, PadSkew>;
 template <class T, int NY, int PROG, bool BAT>
 __global__ __launch_bounds__(64 * plane_nw<PROG>()) void k_plane(const cpx<T> *__restrict__ W, cpx<T> *__restrict__ P,
                                                                long long fs, const cpx<T> *__restrict__ twy,
-                                                               ZConst zc, double *__restrict__ pmax,
+                                                               ZConst zc, ProdLay pl, cpx<T> *__restrict__ probe,
+                                                               double *__restrict__ pmax,
                                                                const int *__restrict__ gate, Batch bt) {
     if constexpr (BAT) {
         W = rebase(bt, 0, W);
         P = rebase(bt, 1, P);
         pmax = rebase(bt, 2, pmax);
         gate = rebase(bt, 3, gate);
+        probe = rebase(bt, 4, probe);
         zc.chi = 1.0 / batch_row(bt)->reynolds_ani;
     }
     if (gate != nullptr && *gate == 0) return;
@@ -173,9 +175,14 @@ __global__ __launch_bounds__(64 * plane_nw<PROG>()) void k_plane(const cpx<T> *_
             for (int i = 0; i < E; i++) v[i] = R[PadSkew::at(t + i * PL_TPL)];
             lsync<true>();
             PlaneFFT<T, NY, -1>::run(v, R, t, twl);
-            cpx<T> *dst = P + (long long)q * fs + plane + c;
+            // the modes the mask keeps (with the 2/3 mask k_z = 0 alone: half the stores)
+            if (lane == 0) probe[q * gridDim.x + blockIdx.x] = v[0];
+            cpx<T> *dst = P + (long long)q * fs + (long long)blockIdx.x * pl.xs + c;
 #pragma unroll
-            for (int i = 0; i < E; i++) dst[2 * (t + i * PL_TPL)] = v[i];
+            for (int i = 0; i < E; i++) {
+                const int r = c < pl.kc ? prod_row(pl, t + i * PL_TPL) : -1;
+                if (r >= 0) dst[r * pl.kp] = v[i];
+            }
         }
     }
 }
@@ -303,12 +310,12 @@ bool plane_rkl_supported(const Grid3 &g) {
 
 template <class T, int NY, bool BAT>
 static int plane_prog(int prog, spk_ctx ctx, const Grid3 &g, const cpx<T> *tw, const cpx<T> *W, cpx<T> *P,
-                      const ZConst &zc, double *pmax, const Batch &bt) {
+                      const ZConst &zc, const ProdLay &pl, cpx<T> *probe, double *pmax, const Batch &bt) {
     const dim3 grid((unsigned)g.nx, 1, nboxes(ctx));
 #define SPK_PL(PR)                                                                                      \
     case PR:                                                                                            \
-        k_plane<T, NY, PR, BAT><<<grid, 64 * plane_nw<PR>(), 0, ctx->stream>>>(W, P, g.ntc, tw, zc, pmax, \
-                                                                                ctx->gate, bt);         \
+        k_plane<T, NY, PR, BAT><<<grid, 64 * plane_nw<PR>(), 0, ctx->stream>>>(W, P, g.ntc, tw, zc, pl, \
+                                                                                probe, pmax, ctx->gate, bt); \
         break;
     switch (prog) {
         SPK_PL(ZP_U)
@@ -324,34 +331,34 @@ static int plane_prog(int prog, spk_ctx ctx, const Grid3 &g, const cpx<T> *tw, c
 
 template <class T, bool BAT>
 static int plane_t(int prog, spk_ctx ctx, const Grid3 &g, const cpx<T> *tw, const cpx<T> *W, cpx<T> *P,
-                   const ZConst &zc, double *pmax, const Batch &bt) {
+                   const ZConst &zc, const ProdLay &pl, cpx<T> *probe, double *pmax, const Batch &bt) {
     switch (g.ny) {
-        case 64: return plane_prog<T, 64, BAT>(prog, ctx, g, tw, W, P, zc, pmax, bt);
-        case 128: return plane_prog<T, 128, BAT>(prog, ctx, g, tw, W, P, zc, pmax, bt);
-        case 256: return plane_prog<T, 256, BAT>(prog, ctx, g, tw, W, P, zc, pmax, bt);
-        case 512: return plane_prog<T, 512, BAT>(prog, ctx, g, tw, W, P, zc, pmax, bt);
+        case 64: return plane_prog<T, 64, BAT>(prog, ctx, g, tw, W, P, zc, pl, probe, pmax, bt);
+        case 128: return plane_prog<T, 128, BAT>(prog, ctx, g, tw, W, P, zc, pl, probe, pmax, bt);
+        case 256: return plane_prog<T, 256, BAT>(prog, ctx, g, tw, W, P, zc, pl, probe, pmax, bt);
+        case 512: return plane_prog<T, 512, BAT>(prog, ctx, g, tw, W, P, zc, pl, probe, pmax, bt);
         default: set_error("plane kernel: NY=%d not supported", g.ny); return SPK_ERR_ARG;
     }
 }
 
 int launch_plane(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int prog, const void *W, void *P,
-                 const ZConst &zc, double *pmax) {
+                 const ZConst &zc, const ProdLay &pl, void *probe, double *pmax) {
     SPK_REQUIRE(plane_supported(g, prog), SPK_ERR_STATE, "plane kernel: grid %dx%dx%d, program %d not supported",
                 g.nx, g.ny, g.nz, prog);
     Batch bt;
-    SPK_TRY(make_batch(ctx, {W, P, pmax, ctx->gate}, &bt));
+    SPK_TRY(make_batch(ctx, {W, P, pmax, ctx->gate, probe}, &bt));
     if (tw.prec == SPK_F64) {
         const cpx<double> *t = reinterpret_cast<const cpx<double> *>(tw.d) + tw.off_y;
         const cpx<double> *w = (const cpx<double> *)W;
         cpx<double> *p = (cpx<double> *)P;
-        return bt.rows ? plane_t<double, true>(prog, ctx, g, t, w, p, zc, pmax, bt)
-                       : plane_t<double, false>(prog, ctx, g, t, w, p, zc, pmax, bt);
+        return bt.rows ? plane_t<double, true>(prog, ctx, g, t, w, p, zc, pl, (cpx<double> *)probe, pmax, bt)
+                       : plane_t<double, false>(prog, ctx, g, t, w, p, zc, pl, (cpx<double> *)probe, pmax, bt);
     }
     const cpx<float> *t = reinterpret_cast<const cpx<float> *>(tw.d) + tw.off_y;
     const cpx<float> *w = (const cpx<float> *)W;
     cpx<float> *p = (cpx<float> *)P;
-    return bt.rows ? plane_t<float, true>(prog, ctx, g, t, w, p, zc, pmax, bt)
-                   : plane_t<float, false>(prog, ctx, g, t, w, p, zc, pmax, bt);
+    return bt.rows ? plane_t<float, true>(prog, ctx, g, t, w, p, zc, pl, (cpx<float> *)probe, pmax, bt)
+                   : plane_t<float, false>(prog, ctx, g, t, w, p, zc, pl, (cpx<float> *)probe, pmax, bt);
 }
 
 template <class T, bool BAT>

@@ -122,14 +122,15 @@ struct ZRow {
     }
     template <class TO>
     __device__ static __forceinline__ void r2c_tw(cpx<T> (&v)[E], bool active, cpx<TO> *dst, cpx<T> *L, int t,
-                                                  const RowTw &rt) {
+                                                  const RowTw &rt, int kc) {
         static_assert(REG, "r2c_tw needs REG");
-        r2c_impl(v, active, dst, L, t, nullptr, nullptr, &rt);
+        r2c_impl(v, active, dst, L, t, nullptr, nullptr, &rt, kc);
     }
     template <class TO>
     __device__ static __forceinline__ void r2c_impl(cpx<T> (&v)[E], bool active, cpx<TO> *dst, cpx<T> *L, int t,
                                                     const cpx<T> *__restrict__ tw_nz,
-                                                    const cpx<T> *__restrict__ tw_m, const RowTw *rt) {
+                                                    const cpx<T> *__restrict__ tw_m, const RowTw *rt, int kc = M + 1) {
+        // kc: the first kc of the M + 1 modes are stored
         if constexpr (REG) FFTF::run_tw(v, L, t, rt->f);
         else FFTF::run(v, L, t, tw_m);
 #pragma unroll
@@ -146,9 +147,9 @@ struct ZRow {
                 cpx<T> w;
                 if constexpr (REG) w = rt->wz[i];
                 else w = tw_nz[k];
-                dst[k] = cconv<TO>(ev + cmul(od, w));
+                if (k < kc) dst[k] = cconv<TO>(ev + cmul(od, w));
             }
-            if (t == 0) {
+            if (t == 0 && M < kc) {
                 const cpx<T> z0 = L[PAD::at(0)];
                 dst[M] = cconv<TO>(cpx<T>{z0.x - z0.y, (T)0});
             }

@@ -648,12 +648,13 @@ int launch_pass_y_rkl(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, 
 int launch_fwdx_rkl2(spk_ctx ctx, int bulk, int nx, const void *Q, void *U, void *Uc0, void *Uc1, void *dU0, void *W,
                      const RklConst &c, int stage, double mu, double nu, double dtmut, double gdt, int inv,
                      double scale, const void *tw, const RklPlan *plan, const TimeState *ts);
-int launch_fwdx_epilogue(spk_ctx ctx, int bulk, int nx, int ly, int mode, int ef, const void *P, void *U, void *S,
-                         void *W, const FusedConst &fc, const void *tw, const TimeState *ts, int ngroups);
+int launch_fwdx_epilogue(spk_ctx ctx, int bulk, int nx, int ly, int mode, int ef, const void *P, const void *probe,
+                         void *U, void *S, void *W, const FusedConst &fc, const void *tw, const TimeState *ts,
+                         int ngroups);
 bool plane_supported(const Grid3 &g, int prog);
 bool plane_rkl_supported(const Grid3 &g);
 int launch_plane(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int prog, const void *W, void *P,
-                 const ZConst &zc, double *pmax);
+                 const ZConst &zc, const ProdLay &pl, void *probe, double *pmax);
 int launch_plane_rkl(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const void *G, const void *Breal, void *Q,
                      const KGeom &kg, const ZConst &zc);
 }  // namespace spk
@@ -678,6 +679,7 @@ struct spk_solver_s {
     // RHS program
     int zprog, nin, nout, oT, oE, oQ, oA;
     InvProg inv;
+    ProdLay pl;  // layout of the products P
     // RKL2 program (anisotropic conduction of theta)
     int rkl_aniso;
     InvProg inv_rkl;
@@ -686,6 +688,7 @@ struct spk_solver_s {
     cpx<double> *U, *S, *dU;
     double *realbuf;
     void *W, *P, *W2, *P2;
+    void *probe;        // [nout][NX] bulk: mode (k_y, k_z) = 0 of the products at each x
     void *Breal;        // real-space B rows (padded, bulk precision), made once per RKL2 cycle
     cpx<double> *diag;  // 6 FP64 fields of scratch for the timevar diagnostics, allocated at first use
     int rkl_cache_b;    // B is not an sts variable: its real-space rows stay valid for a whole cycle
@@ -736,6 +739,34 @@ KGeom kgeom(const spk_solver_s *s, double kxshift) {
 
 unsigned nblk(long long n) { return (unsigned)((n + 255) / 256); }
 
+// the whole spectrum, no mode left out
+ProdLay full_lay(const Grid3 &g) { return ProdLay{g.nzh, g.nzh, g.ny, 0, (long long)g.ny * g.nzh}; }
+
+// the columns the 2/3 mask keeps (kvec_at's comparisons); rows pitched to 128
+// bytes unless they are shorter than half of that
+ProdLay masked_lay(const Grid3 &g, const KGeom &k, size_t esz) {
+    ProdLay l = full_lay(g);
+    if (!k.antialias) return l;
+    l.kc = 0;
+    while (l.kc < g.nzh && !(fabs(k.kfz * (double)l.kc) > k.thz)) l.kc++;
+    l.jc = 0;
+    while (l.jc + 1 <= g.ny / 2 && !(fabs(k.kfy * (double)(l.jc + 1)) > k.thy)) l.jc++;
+    if (l.kc < 1 || 2 * l.jc + 1 > g.ny) return full_lay(g);
+    l.nskip = g.ny - (2 * l.jc + 1);
+    const int al = (int)(128 / esz);
+    l.kp = l.kc <= al / 2 ? l.kc : (l.kc + al - 1) / al * al;
+    if (l.kp > g.nzh) l.kp = g.nzh;
+    // planes an odd number of 4 KB apart: the points of an x line then spread over
+    // the memory channels
+    const long long page = (long long)(4096 / esz), full = (long long)g.ny * l.kp;
+    l.xs = full;
+    if (full >= 4 * page) {
+        const long long pages = ((full + page - 1) / page) | 1;
+        if (pages * page <= (long long)g.ny * g.nzh) l.xs = pages * page;
+    }
+    return l;
+}
+
 // ---- dispatchers over the grid size ----
 
 template <class T>
@@ -768,10 +799,10 @@ int launch_inv_x(spk_solver s, const InvProg &prog, int nslots, void *W, double 
 template <class T, int NZ, bool BAT>
 int launch_zmid_prog(int prog, dim3 grid, int nt, hipStream_t st, const cpx<T> *w, const cpx<T> *wr, cpx<T> *pp,
                      long long nrows, long long ntc, const cpx<T> *tz, const cpx<T> *tm, const ZConst &zc,
-                     double *pmax, const int *gate, const Batch &bt) {
+                     const ProdLay &pl, int ny, double *pmax, const int *gate, const Batch &bt) {
 #define SPK_ZP(PR)                                                                                           \
     case PR:                                                                                                 \
-        k_zmid<T, NZ, PR, BAT><<<grid, nt, 0, st>>>(w, wr, pp, nrows, ntc, tz, tm, zc, pmax, gate, bt); \
+        k_zmid<T, NZ, PR, BAT><<<grid, nt, 0, st>>>(w, wr, pp, nrows, ntc, tz, tm, zc, pl, ny, pmax, gate, bt); \
         break;
     switch (prog) {
         SPK_ZP(ZP_U)
@@ -789,7 +820,8 @@ int launch_zmid_prog(int prog, dim3 grid, int nt, hipStream_t st, const cpx<T> *
 }
 
 template <class T, int NZ>
-int launch_zmid_nz(spk_solver s, int prog, const void *W, void *P, double *pmax, unsigned *nblocks_out) {
+int launch_zmid_nz(spk_solver s, int prog, const void *W, void *P, const ProdLay &pl, double *pmax,
+                   unsigned *nblocks_out) {
     constexpr int M = NZ / 2;
     constexpr int RW = zmid_rw<T>(M);
     constexpr int NT = RW * (M / zmid_e<T>(M));
@@ -806,24 +838,25 @@ int launch_zmid_nz(spk_solver s, int prog, const void *W, void *P, double *pmax,
     const dim3 grid(nb, 1, nboxes(s->ctx));
     if (bt.rows)
         return launch_zmid_prog<T, NZ, true>(prog, grid, NT, s->ctx->stream, w, wr, pp, nrows, s->g.ntc, tz, tm, zc,
-                                             pmax, s->ctx->gate, bt);
+                                             pl, s->g.ny, pmax, s->ctx->gate, bt);
     return launch_zmid_prog<T, NZ, false>(prog, grid, NT, s->ctx->stream, w, wr, pp, nrows, s->g.ntc, tz, tm, zc,
-                                          pmax, s->ctx->gate, bt);
+                                          pl, s->g.ny, pmax, s->ctx->gate, bt);
 }
 
 template <class T>
-int launch_zmid(spk_solver s, int prog, const void *W, void *P, double *pmax, unsigned *nblocks_out) {
+int launch_zmid(spk_solver s, int prog, const void *W, void *P, const ProdLay &pl, double *pmax,
+                unsigned *nblocks_out) {
     switch (s->g.nz) {
-        case 2: return launch_zmid_nz<T, 2>(s, prog, W, P, pmax, nblocks_out);
-        case 4: return launch_zmid_nz<T, 4>(s, prog, W, P, pmax, nblocks_out);
-        case 8: return launch_zmid_nz<T, 8>(s, prog, W, P, pmax, nblocks_out);
-        case 16: return launch_zmid_nz<T, 16>(s, prog, W, P, pmax, nblocks_out);
-        case 32: return launch_zmid_nz<T, 32>(s, prog, W, P, pmax, nblocks_out);
-        case 64: return launch_zmid_nz<T, 64>(s, prog, W, P, pmax, nblocks_out);
-        case 128: return launch_zmid_nz<T, 128>(s, prog, W, P, pmax, nblocks_out);
-        case 256: return launch_zmid_nz<T, 256>(s, prog, W, P, pmax, nblocks_out);
-        case 512: return launch_zmid_nz<T, 512>(s, prog, W, P, pmax, nblocks_out);
-        case 1024: return launch_zmid_nz<T, 1024>(s, prog, W, P, pmax, nblocks_out);
+        case 2: return launch_zmid_nz<T, 2>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 4: return launch_zmid_nz<T, 4>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 8: return launch_zmid_nz<T, 8>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 16: return launch_zmid_nz<T, 16>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 32: return launch_zmid_nz<T, 32>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 64: return launch_zmid_nz<T, 64>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 128: return launch_zmid_nz<T, 128>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 256: return launch_zmid_nz<T, 256>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 512: return launch_zmid_nz<T, 512>(s, prog, W, P, pl, pmax, nblocks_out);
+        case 1024: return launch_zmid_nz<T, 1024>(s, prog, W, P, pl, pmax, nblocks_out);
         default: set_error("NZ=%d unsupported", s->g.nz); return SPK_ERR_ARG;
     }
 }
@@ -880,15 +913,15 @@ int rhs_mid(spk_solver s, bool with_max) {
     s->fused_w_ok = false;  // W no longer holds the last fused step's inverse x pass as it left it
     double *pm = with_max ? s->pmax : nullptr;
     if (plane_front(s)) {
-        SPK_TRY(launch_plane(s->ctx, g, s->twb, s->zprog, s->W, s->P, zconst(s), pm));
+        SPK_TRY(launch_plane(s->ctx, g, s->twb, s->zprog, s->W, s->P, zconst(s), s->pl, s->probe, pm));
         s->zmid_blocks = g.nx;
         return SPK_OK;
     }
     PassArgs a{s->W, s->W, s->nin, g.ntc, g.ntc, 1.0};
     SPK_TRY(launch_pass_y(s->ctx, g, s->twb, +1, s->bulk, s->bulk, a));
     unsigned nb = 0;
-    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, s->zprog, s->W, s->P, pm, &nb));
-    else SPK_TRY(launch_zmid<float>(s, s->zprog, s->W, s->P, pm, &nb));
+    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, s->zprog, s->W, s->P, s->pl, pm, &nb));
+    else SPK_TRY(launch_zmid<float>(s, s->zprog, s->W, s->P, s->pl, pm, &nb));
     s->zmid_blocks = (int)nb;
     return SPK_OK;
 }
@@ -917,6 +950,7 @@ EpiConst make_epi(spk_solver s, double kxshift, double gam, double xi) {
     c.oT = s->oT; c.oE = s->oE; c.oQ = s->oQ; c.oA = s->oA;
     c.gam = gam;
     c.xi = xi;
+    c.pl = s->pl;
     return c;
 }
 
@@ -924,9 +958,8 @@ EpiConst make_epi(spk_solver s, double kxshift, double gam, double xi) {
 int rhs_back(spk_solver s, double kxshift, int mode, double gam, double xi) {
     const Grid3 &g = s->g;
     if (s->nout > 0) {
-        PassArgs a{s->P, s->P, s->nout, g.ntc, g.ntc, 1.0};
-        if (!plane_front(s)) SPK_TRY(launch_pass_y(s->ctx, g, s->twb, -1, s->bulk, s->bulk, a));
-        SPK_TRY(launch_pass_x(s->ctx, g, s->twb, -1, s->bulk, s->bulk, a));
+        if (!plane_front(s)) SPK_TRY(launch_pass_y_products(s->ctx, g, s->twb, s->P, s->nout, s->pl, s->probe));
+        SPK_TRY(launch_pass_x_products(s->ctx, g, s->twb, s->P, s->nout, s->pl));
     }
     const EpiConst c = make_epi(s, kxshift, gam, xi);
     if (s->bulk == SPK_F64) return launch_epilogue<double>(s, c, mode);
@@ -956,8 +989,7 @@ int fused_groups(spk_solver s) {
 
 int rhs_back_fused(spk_solver s, int mode, double gam, double xi, int project, int inv) {
     const Grid3 &g = s->g;
-    PassArgs a{s->P, s->P, s->nout, g.ntc, g.ntc, 1.0};
-    if (!plane_front(s)) SPK_TRY(launch_pass_y(s->ctx, g, s->twb, -1, s->bulk, s->bulk, a));
+    if (!plane_front(s)) SPK_TRY(launch_pass_y_products(s->ctx, g, s->twb, s->P, s->nout, s->pl, s->probe));
     FusedConst fc;
     memset(&fc, 0, sizeof(fc));
     fc.e = make_epi(s, 0.0, gam, xi);
@@ -969,8 +1001,8 @@ int rhs_back_fused(spk_solver s, int mode, double gam, double xi, int project, i
     fc.cu = mode == 2 ? gammaRK[0] : 0.0;
     fc.cs = mode == 2 ? gammaRK[0] + xiRK[0] : (mode == 3 ? xiRK[1] : 0.0);
     const void *tw = (const char *)s->twb.d + (size_t)s->twb.off_x * (s->bulk == SPK_F64 ? 16 : 8);
-    return launch_fwdx_epilogue(s->ctx, s->bulk, g.nx, s->ly, mode, s->fused_ef, s->P, s->U, s->S, s->W, fc, tw,
-                                s->ts, fused_groups(s));
+    return launch_fwdx_epilogue(s->ctx, s->bulk, g.nx, s->ly, mode, s->fused_ef, s->P, s->probe, s->U, s->S, s->W,
+                                fc, tw, s->ts, fused_groups(s));
 }
 
 // inverse y pass + fused z kernel from a W that already holds the inverse x pass
@@ -1143,8 +1175,8 @@ int rkl2_front(spk_solver s) {
     else SPK_TRY(launch_inv_x<float>(s, s->inv_rkl, 6, s->W2, ks));
     PassArgs a{s->W2, s->W2, 6, g.ntc, g.ntc, 1.0};
     SPK_TRY(launch_pass_y(s->ctx, g, s->twb, +1, s->bulk, s->bulk, a));
-    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G, s->W2, s->P2, nullptr, nullptr));
-    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G, s->W2, s->P2, nullptr, nullptr));
+    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
+    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
     PassArgs b{s->P2, s->P2, 3, g.ntc, g.ntc, 1.0};
     SPK_TRY(launch_pass_y(s->ctx, g, s->twb, -1, s->bulk, s->bulk, b));
     SPK_TRY(launch_pass_x(s->ctx, g, s->twb, -1, s->bulk, s->bulk, b));
@@ -1186,8 +1218,8 @@ int rkl2_front_cached(spk_solver s) {
     else SPK_TRY(launch_inv_x<float>(s, s->inv_rkl_g, 3, wg, ks));
     PassArgs a{wg, wg, 3, g.ntc, g.ntc, 1.0};
     SPK_TRY(launch_pass_y(s->ctx, g, s->twb, +1, s->bulk, s->bulk, a));
-    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, nullptr, nullptr));
-    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, nullptr, nullptr));
+    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
+    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
     PassArgs b{s->P2, s->P2, 3, g.ntc, g.ntc, 1.0};
     SPK_TRY(launch_pass_y(s->ctx, g, s->twb, -1, s->bulk, s->bulk, b));
     SPK_TRY(launch_pass_x(s->ctx, g, s->twb, -1, s->bulk, s->bulk, b));
@@ -1217,8 +1249,8 @@ int rkl2_front_fused(spk_solver s, bool with_inv_x) {
     const KGeom kg = kgeom(s, 0.0);
     if (plane_rkl(s)) return launch_plane_rkl(s->ctx, g, s->twb, wg, s->Breal, s->P2, kg, zconst(s));
     SPK_TRY(launch_pass_y_rkl(s->ctx, g, s->twb, +1, wg, kg));
-    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, nullptr, nullptr));
-    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, nullptr, nullptr));
+    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
+    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
     return launch_pass_y_rkl(s->ctx, g, s->twb, -1, s->P2, kg);
 }
 
@@ -1349,25 +1381,26 @@ int tune_fused(spk_solver s) {
         SPK_HIP(hipEventElapsedTime(ms, e0, e1));
         return SPK_OK;
     };
-    float best = 1e30f, t_unf = 0.f, t_cl = 0.f;
+    // The choice is the tile count's unless another one is clearly (15%) faster,
+    // so that solvers of one shape make the same choice and give the same bits:
+    // 8 points per thread where that leaves a block for most CUs (measured per
+    // stage, us, 4 / 8 points: 64^3 MHD FP64 22 / 29 with 66 blocks, 1024x32x32
+    // 111 / 97 with 272).
+    const long long tiles8 = ((long long)g.ny * g.nzh + fx_tcols(g.nx, 8) - 1) / fx_tcols(g.nx, 8);
+    float t_fx[2] = {0.f, 0.f}, t_unf = 0.f, t_cl = 0.f;
     int rc = SPK_OK;
-    for (int ef : {4, 8}) {
-        float ms = 0.f;
+    for (int k = 0; k < 2 && rc == SPK_OK; k++)
         rc = time_it([&] {
-            return launch_fwdx_epilogue(s->ctx, s->bulk, g.nx, s->ly, 2, ef, s->P, s->U, s->S, s->W, fc, tw, s->ts,
-                                        fused_groups(s));
-        }, &ms);
-        if (rc != SPK_OK) break;
-        if (ms < best) {
-            best = ms;
-            s->fused_ef = ef;
-        }
-    }
+            return launch_fwdx_epilogue(s->ctx, s->bulk, g.nx, s->ly, 2, 4 + 4 * k, s->P, s->probe, s->U, s->S, s->W, fc,
+                                        tw, s->ts, fused_groups(s));
+        }, &t_fx[k]);
+    int pick = tiles8 * fused_groups(s) >= 192 ? 1 : 0;
+    if (t_fx[1 - pick] < 0.85f * t_fx[pick]) pick = 1 - pick;
+    s->fused_ef = 4 + 4 * pick;
     if (rc == SPK_OK) {
         const EpiConst c = make_epi(s, 0.0, 0.0, 0.0);
-        PassArgs ap{s->P, s->P, s->nout, g.ntc, g.ntc, 1.0};
         rc = time_it([&] {
-            SPK_TRY(launch_pass_x(s->ctx, g, s->twb, -1, s->bulk, s->bulk, ap));
+            SPK_TRY(launch_pass_x_products(s->ctx, g, s->twb, s->P, s->nout, s->pl));
             SPK_TRY(s->bulk == SPK_F64 ? launch_epilogue<double>(s, c, 2) : launch_epilogue<float>(s, c, 2));
             return s->bulk == SPK_F64 ? launch_inv_x<double>(s, s->inv, s->nin, s->W, 0.0)
                                       : launch_inv_x<float>(s, s->inv, s->nin, s->W, 0.0);
@@ -1377,7 +1410,7 @@ int tune_fused(spk_solver s) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     SPK_TRY(rc);
-    s->fused_faster = best < t_unf + t_cl / 3.0f;
+    s->fused_faster = 0.85f * t_fx[pick] < t_unf + t_cl / 3.0f;
     s->fused_ef_auto = s->fused_ef;
     return SPK_OK;
 }
@@ -1438,7 +1471,7 @@ int step_fused(spk_solver s, bool w_valid) {
 void free_all(spk_solver s) {
     void *bufs[] = {s->U,    s->S,    s->dU,   s->realbuf,  s->W,  s->P,    s->W2,   s->P2,  s->Breal,     s->diag,
                     s->rUc0, s->rUc1, s->rdU0, s->rkl_plan, s->ts, s->pmax, s->part, s->res, s->spec, s->force_idx,
-                    s->force_val};
+                    s->force_val, s->probe};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     twiddles_destroy(&s->twb);
@@ -1585,6 +1618,10 @@ int create(spk_ctx ctx, const spk_params *pin, int bulk, spk_solver s) {
     SPK_TRY(dalloc(&s->realbuf, f64 * s->nf));
     SPK_TRY(dalloc(&s->W, fb * (s->nin > 0 ? s->nin : 1)));
     SPK_TRY(dalloc(&s->P, fb * (s->nout > 0 ? s->nout : 1)));
+    s->pl = masked_lay(s->g, kg, esize(bulk));
+    const size_t probe_bytes = esize(bulk) * (size_t)p.nx * (s->nout > 0 ? s->nout : 1);
+    SPK_TRY(dalloc(&s->probe, probe_bytes));
+    SPK_HIP(hipMemsetAsync(s->probe, 0, probe_bytes, ctx->stream));
     if (s->rkl_aniso) {
         SPK_TRY(dalloc(&s->W2, fb * 6));
         SPK_TRY(dalloc(&s->P2, fb * 3));
@@ -2296,32 +2333,17 @@ extern "C" int spk_kernel_timings(spk_solver s, int reps, double *out_ms, int ca
             if (rc) break;
             unsigned nb = 0;
             rc = timed(2, [&] {
-                return s->bulk == SPK_F64 ? launch_zmid<double>(s, s->zprog, s->W, s->P, s->pmax, &nb)
-                                          : launch_zmid<float>(s, s->zprog, s->W, s->P, s->pmax, &nb);
+                return s->bulk == SPK_F64 ? launch_zmid<double>(s, s->zprog, s->W, s->P, s->pl, s->pmax, &nb)
+                                          : launch_zmid<float>(s, s->zprog, s->W, s->P, s->pl, s->pmax, &nb);
             });
             if (rc) break;
             s->zmid_blocks = (int)nb;
-            PassArgs ap{s->P, s->P, s->nout, g.ntc, g.ntc, 1.0};
-            rc = timed(3, [&] { return launch_pass_y(s->ctx, g, s->twb, -1, s->bulk, s->bulk, ap); });
+            rc = timed(3, [&] { return launch_pass_y_products(s->ctx, g, s->twb, s->P, s->nout, s->pl, s->probe); });
             if (rc) break;
-            rc = timed(4, [&] { return launch_pass_x(s->ctx, g, s->twb, -1, s->bulk, s->bulk, ap); });
+            rc = timed(4, [&] { return launch_pass_x_products(s->ctx, g, s->twb, s->P, s->nout, s->pl); });
             if (rc) break;
         }
-        EpiConst c;
-        memset(&c, 0, sizeof(c));
-        c.kg = kgeom(s, ks);
-        c.ntc = g.ntc;
-        c.stratification = s->p.stratification;
-        c.sd = s->p.strat_direction;
-        c.shearing = s->p.shearing;
-        c.rot_active = s->p.rotating && s->p.shearing;
-        c.aniso_rhs = s->aniso_rhs;
-        c.diff_mask = s->diff_mask;
-        c.nu = s->p.nu; c.nu_m = s->p.nu_m; c.nu_th = s->p.nu_th; c.N2 = s->p.N2;
-        c.shear = s->p.shear; c.omega = s->p.omega;
-        c.oT = s->oT; c.oE = s->oE; c.oQ = s->oQ; c.oA = s->oA;
-        c.gam = 0.0;  // U is restored from the copy after timing
-        c.xi = 0.0;
+        const EpiConst c = make_epi(s, ks, 0.0, 0.0);  // U is restored from the copy after timing
         rc = timed(5, [&] {
             return s->bulk == SPK_F64 ? launch_epilogue<double>(s, c, 2) : launch_epilogue<float>(s, c, 2);
         });
@@ -2336,13 +2358,13 @@ extern "C" int spk_kernel_timings(spk_solver s, int reps, double *out_ms, int ca
             FusedConst fc;
             memset(&fc, 0, sizeof(fc));
             fc.e = c;
-            fc.project = 0;
+                    fc.project = 0;
             fc.inv = 1;
             fc.scale = 1.0 / ((double)g.nx * g.ny * g.nz);
             const void *tw = (const char *)s->twb.d + (size_t)s->twb.off_x * (s->bulk == SPK_F64 ? 16 : 8);
             rc = timed(8, [&] {
-                return launch_fwdx_epilogue(s->ctx, s->bulk, g.nx, s->ly, 2, s->fused_ef, s->P, s->U, s->S, s->W, fc,
-                                            tw, s->ts, fused_groups(s));
+                return launch_fwdx_epilogue(s->ctx, s->bulk, g.nx, s->ly, 2, s->fused_ef, s->P, s->probe, s->U, s->S,
+                                            s->W, fc, tw, s->ts, fused_groups(s));
             });
         }
     } while (0);
@@ -2402,6 +2424,7 @@ void solver_box_row(spk_solver s, BoxRow *row, size_t *sizes) {
     put(SL_UC1, s->rUc1, f64 * s->nsts);
     put(SL_DU0, s->rdU0, f64 * s->nsts);
     put(SL_PLAN, s->rkl_plan, sizeof(RklPlan));
+    put(SL_PROBE, s->probe, esize(s->bulk) * (size_t)s->p.nx * (s->nout > 0 ? s->nout : 1));
     row->nu = s->p.nu;
     row->nu_m = s->p.nu_m;
     row->nu_th = s->p.nu_th;
