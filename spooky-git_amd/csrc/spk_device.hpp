@@ -421,7 +421,7 @@ struct BoxRow {
     char *p[BOX_SLOTS];                   // the box's arrays, by slot
     double nu, nu_m, nu_th, reynolds_ani; // the coefficients a box may set for itself
 };
-constexpr int BATCH_ARGS = 8;
+constexpr int BATCH_ARGS = 9;
 struct Batch {
     const BoxRow *rows;
     signed char slot[BATCH_ARGS];  // -1: the argument is the same for every box

@@ -271,7 +271,16 @@ static int launch_y_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, vo
 #define SPK_YP_CASE(NN)                                                                                     \
     case NN: {                                                                                              \
         constexpr int TC = strided_tcols_t<T>(NN);                                                          \
-        const long long ntiles = ((long long)l.kc * g.nx + TC - 1) / TC;                                    \
+        const long long nc = (long long)l.kc * g.nx;                                                        \
+        if constexpr (TC > 2) {                                                                             \
+            if (l.kc <= 2) { /* a line's points are (almost) contiguous: as the TC = 2 tile of NZ = 2 */    \
+                k_pass_strided<T, NN, -1, 1, 2, true>                                                       \
+                    <<<dim3((unsigned)((nc + 1) / 2), n, nbz), 2 * strided_tpl(NN), 0, ctx->stream>>>(      \
+                        p, p, l.kc, l.kp, l.xs, g.nx, g.ntc, g.ntc, twp, (T)1, ctx->gate, l, pr, bt);       \
+                break;                                                                                      \
+            }                                                                                               \
+        }                                                                                                   \
+        const long long ntiles = (nc + TC - 1) / TC;                                                        \
         dim3 grid((unsigned)ntiles, n, nbz);                                                                \
         k_pass_strided<T, NN, -1, 1, TC, true><<<grid, TC * strided_tpl(NN), 0, ctx->stream>>>(             \
             p, p, l.kc, l.kp, l.xs, g.nx, g.ntc, g.ntc, twp, (T)1, ctx->gate, l, pr, bt);                   \

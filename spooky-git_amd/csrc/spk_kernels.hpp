@@ -60,6 +60,7 @@ struct RklConst {
     int field[8];    // state index of sts variable n
     int kind[8];     // 0: -nu k^2, 1: -nu_m k^2, 2: -nu_th k^2, 3: div of anisotropic flux
     double nu, nu_m, nu_th;
+    ProdLay pl;      // layout of the flux products (fused stage)
 };
 
 // Device-sized RKL2 cycle: the stage count and coefficient table of the
@@ -595,12 +596,16 @@ __device__ __forceinline__ int fx_tile(int b, int nt, int first) {
     tile += first;
     return tile < nt ? tile : tile - nt;
 }
-__device__ __forceinline__ bool fx_masked_tile(const EpiConst &c, int c0, int c1) {
-    int j = c0 / c.kg.nzh;
-    if (c0 - j * c.kg.nzh < c.pl.kc && prod_row(c.pl, j) >= 0) return false;
-    for (j++; j * c.kg.nzh < c1; j++)
-        if (prod_row(c.pl, j) >= 0) return false;
+__device__ __forceinline__ bool fx_masked_tile(const ProdLay &l, int nzh, int c0, int c1) {
+    int j = c0 / nzh;
+    if (c0 - j * nzh < l.kc && prod_row(l, j) >= 0) return false;
+    for (j++; j * nzh < c1; j++)
+        if (prod_row(l, j) >= 0) return false;
     return true;
+}
+// the first tile past the masked rows
+__device__ __forceinline__ int fx_first_tile(const ProdLay &l, int nzh, int tc) {
+    return l.nskip > 0 ? (l.jc + 1 + l.nskip) * nzh / tc : 0;
 }
 
 // vmcnt(0) and lgkmcnt(0) waits (gfx9 s_waitcnt encodings; other counters at
@@ -1039,15 +1044,13 @@ __global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilog
     const int cl = tid % TC;
     int t = tid / TC;
     const int ncols = fc.e.kg.ny * fc.e.kg.nzh;
-    // the first tile past the masked rows
-    const int first = fc.e.pl.nskip > 0 ? (fc.e.pl.jc + 1 + fc.e.pl.nskip) * fc.e.kg.nzh / TC : 0;
-    const int c0 = fx_tile(blockIdx.x, gridDim.x, first) * TC;
+    const int c0 = fx_tile(blockIdx.x, gridDim.x, fx_first_tile(fc.e.pl, fc.e.kg.nzh, TC)) * TC;
     int col = c0 + cl < ncols ? c0 + cl : ncols - 1;
     cpx<T> *ldsc = lds + cl * LL;
     // group: 0 velocity (+ temperature with STRAT), then magnetic (MHD), then
     // temperature (boussinesq without STRAT)
     const int g = blockIdx.y;
-    if (fx_masked_tile(fc.e, c0, c0 + TC < ncols ? c0 + TC : ncols)) {
+    if (fx_masked_tile(fc.e.pl, fc.e.kg.nzh, c0, c0 + TC < ncols ? c0 + TC : ncols)) {
         if (g == 0)
             fx_masked<T, N, LY, MODE, EF, STRAT && L::BOUSS ? 3 : 0>(probe, U, W, fc, tw, twl, ldsc, ts, tid, NT, t, col);
         else if (L::MHD && g == 1)

@@ -192,14 +192,15 @@ __global__ __launch_bounds__(64 * plane_nw<PROG>()) void k_plane(const cpx<T> *_
 // combined into H.  G: slots A, B; Br: B's real-space rows (3 slots); Q: Y, H.
 template <class T, int NY, bool BAT>
 __global__ __launch_bounds__(192) void k_plane_rkl(const cpx<T> *__restrict__ G, const cpx<T> *__restrict__ Br,
-                                                  cpx<T> *__restrict__ Q, long long fs, KGeom kg,
-                                                  const cpx<T> *__restrict__ twy, ZConst zc,
+                                                  cpx<T> *__restrict__ Q, long long fs, KGeom kg, ProdLay pl,
+                                                  cpx<T> *__restrict__ probe, const cpx<T> *__restrict__ twy, ZConst zc,
                                                   const int *__restrict__ gate, Batch bt) {
     if constexpr (BAT) {
         G = rebase(bt, 0, G);
         Br = rebase(bt, 1, Br);
         Q = rebase(bt, 2, Q);
         gate = rebase(bt, 3, gate);
+        probe = rebase(bt, 4, probe);
         zc.chi = 1.0 / batch_row(bt)->reynolds_ani;
     }
     if (gate != nullptr && *gate == 0) return;
@@ -275,10 +276,16 @@ __global__ __launch_bounds__(192) void k_plane_rkl(const cpx<T> *__restrict__ G,
     for (int i = 0; i < E; i++) v[i] = R[PadSkew::at(t + i * PL_TPL)];
     lsync<true>();
     PlaneFFT<T, NY, -1>::run(v, R, t, twl);
+    // the modes the mask keeps
+    auto put = [&](cpx<T> *dst, int n, cpx<T> x) {
+        const int r = c < pl.kc ? prod_row(pl, n) : -1;
+        if (r >= 0) dst[r * pl.kp] = x;
+    };
     if (w == 0) {
-        cpx<T> *dst = Q + plane + c;
+        cpx<T> *dst = Q + (long long)blockIdx.x * pl.xs + c;
 #pragma unroll
-        for (int i = 0; i < E; i++) dst[2 * (t + i * PL_TPL)] = v[i];
+        for (int i = 0; i < E; i++) put(dst, t + i * PL_TPL, v[i]);
+        if (lane == 0) probe[blockIdx.x] = v[0];
     } else if (w == 2) {
         lsync<true>();
 #pragma unroll
@@ -287,12 +294,14 @@ __global__ __launch_bounds__(192) void k_plane_rkl(const cpx<T> *__restrict__ G,
     __syncthreads();
     if (w == 1) {
         const cpx<T> *Rz = reg + (4 + c) * LL;
-        cpx<T> *dst = Q + fs + plane + c;
+        cpx<T> *dst = Q + fs + (long long)blockIdx.x * pl.xs + c;
 #pragma unroll
         for (int i = 0; i < E; i++) {
             const T ky = ky_at(t + i * PL_TPL);
             const cpx<T> z = Rz[PadSkew::at(t + i * PL_TPL)];
-            dst[2 * (t + i * PL_TPL)] = cpx<T>{ky * v[i].x + z.x, ky * v[i].y + z.y};
+            const cpx<T> h = {ky * v[i].x + z.x, ky * v[i].y + z.y};
+            put(dst, t + i * PL_TPL, h);
+            if (i == 0 && lane == 0) probe[gridDim.x + blockIdx.x] = h;
         }
     }
 }
@@ -363,13 +372,14 @@ int launch_plane(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int prog, cons
 
 template <class T, bool BAT>
 static int plane_rkl_t(spk_ctx ctx, const Grid3 &g, const cpx<T> *tw, const cpx<T> *G, const cpx<T> *Br,
-                       cpx<T> *Q, const KGeom &kg, const ZConst &zc, const Batch &bt) {
+                       cpx<T> *Q, const KGeom &kg, const ProdLay &pl, cpx<T> *probe, const ZConst &zc,
+                       const Batch &bt) {
     const dim3 grid((unsigned)g.nx, 1, nboxes(ctx));
     switch (g.ny) {
-        case 64: k_plane_rkl<T, 64, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, tw, zc, ctx->gate, bt); break;
-        case 128: k_plane_rkl<T, 128, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, tw, zc, ctx->gate, bt); break;
-        case 256: k_plane_rkl<T, 256, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, tw, zc, ctx->gate, bt); break;
-        case 512: k_plane_rkl<T, 512, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, tw, zc, ctx->gate, bt); break;
+        case 64: k_plane_rkl<T, 64, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, pl, probe, tw, zc, ctx->gate, bt); break;
+        case 128: k_plane_rkl<T, 128, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, pl, probe, tw, zc, ctx->gate, bt); break;
+        case 256: k_plane_rkl<T, 256, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, pl, probe, tw, zc, ctx->gate, bt); break;
+        case 512: k_plane_rkl<T, 512, BAT><<<grid, 192, 0, ctx->stream>>>(G, Br, Q, g.ntc, kg, pl, probe, tw, zc, ctx->gate, bt); break;
         default: set_error("plane RKL2 kernel: NY=%d not supported", g.ny); return SPK_ERR_ARG;
     }
     SPK_LAUNCH_CHECK();
@@ -377,24 +387,24 @@ static int plane_rkl_t(spk_ctx ctx, const Grid3 &g, const cpx<T> *tw, const cpx<
 }
 
 int launch_plane_rkl(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const void *G, const void *Breal, void *Q,
-                     const KGeom &kg, const ZConst &zc) {
+                     const KGeom &kg, const ProdLay &pl, void *probe, const ZConst &zc) {
     SPK_REQUIRE(plane_rkl_supported(g), SPK_ERR_STATE, "plane RKL2 kernel: grid %dx%dx%d not supported", g.nx, g.ny,
                 g.nz);
     SPK_REQUIRE(kg.kxshift == 0.0, SPK_ERR_STATE, "plane RKL2 kernel: sheared wavevectors are not supported");
     Batch bt;
-    SPK_TRY(make_batch(ctx, {G, Breal, Q, ctx->gate}, &bt));
+    SPK_TRY(make_batch(ctx, {G, Breal, Q, ctx->gate, probe}, &bt));
     if (tw.prec == SPK_F64) {
         const cpx<double> *t = reinterpret_cast<const cpx<double> *>(tw.d) + tw.off_y;
         const cpx<double> *gg = (const cpx<double> *)G, *br = (const cpx<double> *)Breal;
         cpx<double> *q = (cpx<double> *)Q;
-        return bt.rows ? plane_rkl_t<double, true>(ctx, g, t, gg, br, q, kg, zc, bt)
-                       : plane_rkl_t<double, false>(ctx, g, t, gg, br, q, kg, zc, bt);
+        return bt.rows ? plane_rkl_t<double, true>(ctx, g, t, gg, br, q, kg, pl, (cpx<double> *)probe, zc, bt)
+                       : plane_rkl_t<double, false>(ctx, g, t, gg, br, q, kg, pl, (cpx<double> *)probe, zc, bt);
     }
     const cpx<float> *t = reinterpret_cast<const cpx<float> *>(tw.d) + tw.off_y;
     const cpx<float> *gg = (const cpx<float> *)G, *br = (const cpx<float> *)Breal;
     cpx<float> *q = (cpx<float> *)Q;
-    return bt.rows ? plane_rkl_t<float, true>(ctx, g, t, gg, br, q, kg, zc, bt)
-                   : plane_rkl_t<float, false>(ctx, g, t, gg, br, q, kg, zc, bt);
+    return bt.rows ? plane_rkl_t<float, true>(ctx, g, t, gg, br, q, kg, pl, (cpx<float> *)probe, zc, bt)
+                   : plane_rkl_t<float, false>(ctx, g, t, gg, br, q, kg, pl, (cpx<float> *)probe, zc, bt);
 }
 
 }  // namespace spk

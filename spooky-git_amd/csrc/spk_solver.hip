@@ -644,10 +644,11 @@ __global__ __launch_bounds__(256) void k_unshear(const cpx<double> *__restrict__
 namespace spk {
 bool fused_supported_nx(int nx);
 bool rkl_fused_supported_nx(int nx);
-int launch_pass_y_rkl(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, void *buf, const KGeom &kg);
+int launch_pass_y_rkl(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, const void *in, void *out,
+                      const KGeom &kg, const ProdLay &pl, void *probe);
 int launch_fwdx_rkl2(spk_ctx ctx, int bulk, int nx, const void *Q, void *U, void *Uc0, void *Uc1, void *dU0, void *W,
                      const RklConst &c, int stage, double mu, double nu, double dtmut, double gdt, int inv,
-                     double scale, const void *tw, const RklPlan *plan, const TimeState *ts);
+                     double scale, const void *tw, const RklPlan *plan, const TimeState *ts, const void *probe);
 int launch_fwdx_epilogue(spk_ctx ctx, int bulk, int nx, int ly, int mode, int ef, const void *P, const void *probe,
                          void *U, void *S, void *W, const FusedConst &fc, const void *tw, const TimeState *ts,
                          int ngroups);
@@ -656,7 +657,7 @@ bool plane_rkl_supported(const Grid3 &g);
 int launch_plane(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int prog, const void *W, void *P,
                  const ZConst &zc, const ProdLay &pl, void *probe, double *pmax);
 int launch_plane_rkl(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const void *G, const void *Breal, void *Q,
-                     const KGeom &kg, const ZConst &zc);
+                     const KGeom &kg, const ProdLay &pl, void *probe, const ZConst &zc);
 }  // namespace spk
 
 // ==========================================================================
@@ -688,7 +689,7 @@ struct spk_solver_s {
     cpx<double> *U, *S, *dU;
     double *realbuf;
     void *W, *P, *W2, *P2;
-    void *probe;        // [nout][NX] bulk: mode (k_y, k_z) = 0 of the products at each x
+    void *probe;        // [nout + 2][NX] bulk: mode (k_y, k_z) = 0 of the products at each x, and of the RKL2 flux
     void *Breal;        // real-space B rows (padded, bulk precision), made once per RKL2 cycle
     cpx<double> *diag;  // 6 FP64 fields of scratch for the timevar diagnostics, allocated at first use
     int rkl_cache_b;    // B is not an sts variable: its real-space rows stay valid for a whole cycle
@@ -1234,37 +1235,42 @@ bool rkl_fused(spk_solver s) {
            s->fused_mode != 0;
 }
 
+// the (k_y, k_z) = 0 modes of the fused RKL2 flux, after those of the products
+void *rkl_probe(spk_solver s) { return (char *)s->probe + (size_t)s->nout * s->p.nx * esize(s->bulk); }
+
 // the part of a fused RKL2 stage before its forward x pass: (stage 1 only) the
-// inverse x pass of i k_x theta and theta, then the inverse y pass that makes
-// the three gradient components, the flux in the z kernel and the forward y
-// pass that folds k_y F_y + k_z F_z into one slot
+// inverse x pass of i k_x theta and theta into W2's first two slots (the later
+// stages' back part writes them), then the inverse y pass that makes the three
+// gradient components (W2's last three slots), the flux in the z kernel and the
+// forward y pass that folds k_y F_y + k_z F_z into one slot
 int rkl2_front_fused(spk_solver s, bool with_inv_x) {
     const Grid3 &g = s->g;
     const size_t fb = (size_t)g.ntc * esize(s->bulk);
     void *wg = (char *)s->W2 + 3 * fb;  // the grad theta slots of the fused z program
     if (with_inv_x) {
-        if (s->bulk == SPK_F64) SPK_TRY(launch_inv_x<double>(s, s->inv_rkl_t, 2, wg, 0.0));
-        else SPK_TRY(launch_inv_x<float>(s, s->inv_rkl_t, 2, wg, 0.0));
+        if (s->bulk == SPK_F64) SPK_TRY(launch_inv_x<double>(s, s->inv_rkl_t, 2, s->W2, 0.0));
+        else SPK_TRY(launch_inv_x<float>(s, s->inv_rkl_t, 2, s->W2, 0.0));
     }
     const KGeom kg = kgeom(s, 0.0);
-    if (plane_rkl(s)) return launch_plane_rkl(s->ctx, g, s->twb, wg, s->Breal, s->P2, kg, zconst(s));
-    SPK_TRY(launch_pass_y_rkl(s->ctx, g, s->twb, +1, wg, kg));
-    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
-    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, full_lay(s->g), nullptr, nullptr));
-    return launch_pass_y_rkl(s->ctx, g, s->twb, -1, s->P2, kg);
+    if (plane_rkl(s))
+        return launch_plane_rkl(s->ctx, g, s->twb, s->W2, s->Breal, s->P2, kg, s->pl, rkl_probe(s), zconst(s));
+    SPK_TRY(launch_pass_y_rkl(s->ctx, g, s->twb, +1, s->W2, wg, kg, s->pl, rkl_probe(s)));
+    if (s->bulk == SPK_F64) SPK_TRY(launch_zmid<double>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, s->pl, nullptr, nullptr));
+    else SPK_TRY(launch_zmid<float>(s, ZP_B | ZP_G | ZP_BR, s->W2, s->P2, s->pl, nullptr, nullptr));
+    return launch_pass_y_rkl(s->ctx, g, s->twb, -1, s->P2, s->P2, kg, s->pl, rkl_probe(s));
 }
 
 // forward x pass of the flux + stage update + (inv) the next stage's inverse x pass
 int rkl2_back_fused(spk_solver s, int stage, double mu, double nu, double dtmut, double gdt, int inv,
                     const RklPlan *plan) {
     const Grid3 &g = s->g;
-    const size_t fb = (size_t)g.ntc * esize(s->bulk);
     RklConst c = s->rkl;
     c.kg = kgeom(s, 0.0);
+    c.pl = s->pl;
     const void *tw = (const char *)s->twb.d + (size_t)s->twb.off_x * esize(s->bulk);
-    return launch_fwdx_rkl2(s->ctx, s->bulk, g.nx, s->P2, s->U, s->rUc0, s->rUc1, s->rdU0, (char *)s->W2 + 3 * fb, c,
-                            stage, mu, nu, dtmut, gdt, inv, 1.0 / ((double)g.nx * g.ny * g.nz), tw, plan,
-                            plan ? s->ts : nullptr);
+    return launch_fwdx_rkl2(s->ctx, s->bulk, g.nx, s->P2, s->U, s->rUc0, s->rUc1, s->rdU0, s->W2, c, stage, mu, nu,
+                            dtmut, gdt, inv, 1.0 / ((double)g.nx * g.ny * g.nz), tw, plan, plan ? s->ts : nullptr,
+                            rkl_probe(s));
 }
 
 int rkl2_cycle(spk_solver s) {
@@ -1619,7 +1625,7 @@ int create(spk_ctx ctx, const spk_params *pin, int bulk, spk_solver s) {
     SPK_TRY(dalloc(&s->W, fb * (s->nin > 0 ? s->nin : 1)));
     SPK_TRY(dalloc(&s->P, fb * (s->nout > 0 ? s->nout : 1)));
     s->pl = masked_lay(s->g, kg, esize(bulk));
-    const size_t probe_bytes = esize(bulk) * (size_t)p.nx * (s->nout > 0 ? s->nout : 1);
+    const size_t probe_bytes = esize(bulk) * (size_t)p.nx * (s->nout + 2);
     SPK_TRY(dalloc(&s->probe, probe_bytes));
     SPK_HIP(hipMemsetAsync(s->probe, 0, probe_bytes, ctx->stream));
     if (s->rkl_aniso) {
@@ -2424,7 +2430,7 @@ void solver_box_row(spk_solver s, BoxRow *row, size_t *sizes) {
     put(SL_UC1, s->rUc1, f64 * s->nsts);
     put(SL_DU0, s->rdU0, f64 * s->nsts);
     put(SL_PLAN, s->rkl_plan, sizeof(RklPlan));
-    put(SL_PROBE, s->probe, esize(s->bulk) * (size_t)s->p.nx * (s->nout > 0 ? s->nout : 1));
+    put(SL_PROBE, s->probe, esize(s->bulk) * (size_t)s->p.nx * (s->nout + 2));
     row->nu = s->p.nu;
     row->nu_m = s->p.nu_m;
     row->nu_th = s->p.nu_th;

@@ -15,6 +15,8 @@ T = 2 * np.pi
 GRIDS = [(32, 16, 4), (32, 4, 32), (64, 8, 2), (32, 32, 16), (64, 2, 8), (32, 64, 64), (128, 16, 128), (32, 128, 2)]
 PHYS = {"hd": dict(), "mhd": dict(mhd=1, nu_m=3e-3), "open": dict(mhd=1, nu_m=3e-3, antialiasing=0),
         "flat": dict(mhd=1, nu_m=3e-3, with2d=1), "bouss": dict(boussinesq=1, nu_th=2e-3),
+        "rkl": dict(mhd=1, nu_m=3e-3, boussinesq=1, stratification=1, strat_direction=2, N2=0.3, OmegaT2=0.5, nu_th=2e-3,
+                    anisotropic_diffusion=1, reynolds_ani=50.0, supertimestepping=1, sts_mask=1 << 6, safety_sts=20),
         "strat": dict(mhd=1, nu_m=3e-3, boussinesq=1, stratification=1, strat_direction=1, N2=0.4, nu_th=2e-3)}
 
 
@@ -34,6 +36,8 @@ def full_state(p, seed):
     """Real noise in every field, rms 0.3: every mode of its spectrum is filled."""
     nf = 3 + 3 * p.get("mhd", 0) + p.get("boussinesq", 0)
     r = 0.3 * np.random.default_rng(seed).standard_normal((nf, p["nx"], p["ny"], p["nz"]))
+    if p.get("anisotropic_diffusion"):
+        r[3:6] = 0.1 * r[3:6] + np.array([1.0, 0.5, -0.7])[:, None, None, None]  # B nowhere 0
     return np.fft.rfftn(r, axes=(1, 2, 3))
 
 
@@ -64,6 +68,20 @@ def test_filled_spectrum_against_oracle(ctx, grid, phys, prec):
             sol.main_loop(3)
             e = relerr(sol.get_fields(), sim.fields)
             assert e < {"f64": 1e-10, "f32": 2e-4}[prec], (fused, points, e)
+    sol.destroy()
+
+
+@pytest.mark.parametrize("grid", [(32, 16, 16), (64, 64, 2), (32, 64, 64)], ids=lambda g: "%dx%dx%d" % g)
+def test_nan_reaches_every_mode_of_theta(ctx, grid):
+    p = params(grid, "rkl")
+    u0 = full_state(p, 5)
+    u0[6, 1, 1, 0] = np.nan
+    sol = spk.Solver(ctx, "f64", **p)
+    sol.set_fields(full_state(p, 5))
+    sol.compute_dt()
+    sol.set_fields(u0)
+    sol.rkl2_cycle()
+    assert np.all(np.isnan(sol.get_fields()[6, 1:, :, :].real))
     sol.destroy()
 
 
