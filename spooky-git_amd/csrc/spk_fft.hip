@@ -195,6 +195,13 @@ static const cpx<T> *tw_ptr(const Twiddles &tw, long long off) {
 // launchers
 // ------------------------------------------------------------------------
 
+// Columns of a tile on grids whose full tiles would leave most CUs without a
+// block: a quarter, in blocks of one wavefront or more (64^3 HD FP64, 3 fields:
+// 51 blocks of 128 columns 7.6 us, 198 of 32 5.4 us); 0: no smaller tile.
+constexpr int small_tcols(int n, int tc) {
+    return n >= 16 && n <= 512 && tc >= 16 && tc / 4 * strided_tpl(n) >= 64 ? tc / 4 : 0;
+}
+
 // plain passes: no pruning
 static const ProdLay NO_PRUNE{0, 0, 0, 0, 0};
 
@@ -219,6 +226,17 @@ static int launch_strided(spk_ctx ctx, int n, long long ncols, long long lstride
             }                                                                                      \
         }                                                                                          \
         const long long ntiles = (ncols * nouter + TC - 1) / TC;                                   \
+        if constexpr (small_tcols(NN, TC) > 0) {                                                   \
+            if (ntiles * a.nfields * nbz < 256) {                                                  \
+                constexpr int TS = small_tcols(NN, TC);                                            \
+                k_pass_strided<T, NN, DIR, AXIS, TS>                                               \
+                    <<<dim3((unsigned)((ncols * nouter + TS - 1) / TS), a.nfields, nbz),           \
+                       TS * strided_tpl(NN), 0, ctx->stream>>>(                                    \
+                        (const cpx<T> *)a.in, (cpx<T> *)a.out, ncols, lstride, ostride, nouter,    \
+                        a.fstride_in, a.fstride_out, twp, (T)a.scale, ctx->gate, NO_PRUNE, nullptr, bt); \
+                break;                                                                             \
+            }                                                                                      \
+        }                                                                                          \
         dim3 grid((unsigned)ntiles, a.nfields, nbz);                                               \
         k_pass_strided<T, NN, DIR, AXIS, TC><<<grid, TC * strided_tpl(NN), 0, ctx->stream>>>(         \
             (const cpx<T> *)a.in, (cpx<T> *)a.out, ncols, lstride, ostride, nouter, a.fstride_in, \
@@ -281,6 +299,16 @@ static int launch_y_products(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, vo
             }                                                                                               \
         }                                                                                                   \
         const long long ntiles = (nc + TC - 1) / TC;                                                        \
+        if constexpr (small_tcols(NN, TC) > 0) {                                                            \
+            if (ntiles * n * nbz < 256) {                                                                   \
+                constexpr int TS = small_tcols(NN, TC);                                                     \
+                k_pass_strided<T, NN, -1, 1, TS, true>                                                      \
+                    <<<dim3((unsigned)((nc + TS - 1) / TS), n, nbz), TS * strided_tpl(NN), 0,               \
+                       ctx->stream>>>(p, p, l.kc, l.kp, l.xs, g.nx, g.ntc, g.ntc, twp, (T)1, ctx->gate, l,  \
+                                      pr, bt);                                                              \
+                break;                                                                                      \
+            }                                                                                               \
+        }                                                                                                   \
         dim3 grid((unsigned)ntiles, n, nbz);                                                                \
         k_pass_strided<T, NN, -1, 1, TC, true><<<grid, TC * strided_tpl(NN), 0, ctx->stream>>>(             \
             p, p, l.kc, l.kp, l.xs, g.nx, g.ntc, g.ntc, twp, (T)1, ctx->gate, l, pr, bt);                   \

@@ -9,7 +9,7 @@ bool fused_supported_nx(int nx) { return nx >= 32 && nx <= 1024 && is_pow2(nx); 
 
 // ef: points per thread of the x line, 4 or 8 (picked by the solver's tile autotune)
 int launch_fwdx_epilogue(spk_ctx ctx, int bulk, int nx, int ly, int mode, int ef, const void *P, const void *probe,
-                         void *U, void *S, void *W, const FusedConst &fc, const void *tw, const TimeState *ts,
+                         void *U, void *S, void *W, const FusedConst &fc, const void *tw, TimeState *ts,
                          int ngroups) {
     Batch bt;
     SPK_TRY(make_batch(ctx, {P, U, S, W, ts, probe}, &bt));

@@ -11,7 +11,7 @@ namespace spk {
 
 template <class T, int N, int LY, int EF, bool STRAT = false>
 static void launch_ly_mode(int mode, dim3 grid, int bs, hipStream_t st, const cpx<T> *P, const cpx<T> *probe, cpx<double> *U,
-                           cpx<T> *S, cpx<T> *W, const FusedConst &fc, const cpx<T> *tw, const TimeState *ts,
+                           cpx<T> *S, cpx<T> *W, const FusedConst &fc, const cpx<T> *tw, TimeState *ts,
                            const Batch &bt) {
     switch (mode) {
         case 1: k_fwdx_epilogue<T, N, LY, 1, EF, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
@@ -24,7 +24,7 @@ static void launch_ly_mode(int mode, dim3 grid, int bs, hipStream_t st, const cp
 // groups in one block (k_fwdx_epilogue's STRAT instantiation)
 template <class T, int N, int LY, int EF>
 static int launch_bouss(int mode, dim3 grid, int bs, hipStream_t st, const cpx<T> *P, const cpx<T> *probe, cpx<double> *U, cpx<T> *S,
-                        cpx<T> *W, const FusedConst &fc, const cpx<T> *tw, const TimeState *ts, const Batch &bt) {
+                        cpx<T> *W, const FusedConst &fc, const cpx<T> *tw, TimeState *ts, const Batch &bt) {
     if (!fc.e.stratification) {
         launch_ly_mode<T, N, LY, EF>(mode, grid, bs, st, P, probe, U, S, W, fc, tw, ts, bt);
         return SPK_OK;
@@ -35,7 +35,7 @@ static int launch_bouss(int mode, dim3 grid, int bs, hipStream_t st, const cpx<T
 
 template <class T, int N, int EF>
 static int launch_n(int ly, int mode, hipStream_t st, const void *P, const void *probe, void *U, void *S, void *W,
-                    const FusedConst &fc, const void *tw, const TimeState *ts, int ngroups, const Batch &bt, unsigned nbz) {
+                    const FusedConst &fc, const void *tw, TimeState *ts, int ngroups, const Batch &bt, unsigned nbz) {
     constexpr int TC = fx_tcols(N, EF);
     const long long ncols = (long long)fc.e.kg.ny * fc.e.kg.nzh;
     dim3 grid((unsigned)((ncols + TC - 1) / TC), ngroups, nbz);
@@ -58,7 +58,7 @@ static int launch_n(int ly, int mode, hipStream_t st, const void *P, const void 
 
 template <class T, int EF>
 static int launch_t(int nx, int ly, int mode, hipStream_t st, const void *P, const void *probe, void *U, void *S, void *W,
-                    const FusedConst &fc, const void *tw, const TimeState *ts, int ngroups, const Batch &bt,
+                    const FusedConst &fc, const void *tw, TimeState *ts, int ngroups, const Batch &bt,
                     unsigned nbz) {
     switch (nx) {
         case 32: return launch_n<T, 32, EF>(ly, mode, st, P, probe, U, S, W, fc, tw, ts, ngroups, bt, nbz);
@@ -74,14 +74,14 @@ static int launch_t(int nx, int ly, int mode, hipStream_t st, const void *P, con
 // the instantiations of one precision and EF points per thread
 template <class T, int EF>
 int launch_fwdx_epilogue_t(spk_ctx ctx, int nx, int ly, int mode, const void *P, const void *probe, void *U, void *S,
-                           void *W, const FusedConst &fc, const void *tw, const TimeState *ts, int ngroups,
+                           void *W, const FusedConst &fc, const void *tw, TimeState *ts, int ngroups,
                            const Batch &bt) {
     return launch_t<T, EF>(nx, ly, mode, ctx->stream, P, probe, U, S, W, fc, tw, ts, ngroups, bt, nboxes(ctx));
 }
 
 #define SPK_FUSED_DECL(NAME)                                                                                     \
     int NAME(spk_ctx ctx, int nx, int ly, int mode, const void *P, const void *probe, void *U, void *S, void *W, \
-             const FusedConst &fc, const void *tw, const TimeState *ts, int ngroups, const Batch &bt)
+             const FusedConst &fc, const void *tw, TimeState *ts, int ngroups, const Batch &bt)
 SPK_FUSED_DECL(launch_fused_f64_4);
 SPK_FUSED_DECL(launch_fused_f64_8);
 SPK_FUSED_DECL(launch_fused_f32_4);

@@ -37,6 +37,14 @@ struct SolverViews {
 };
 void solver_views(spk_solver s, SolverViews *v);
 
+// clock updates: t += dt (RungeKutta3), step++ (HydroMHDAdvance), snapshot clock
+// of CheckSnapshot (check_output.cu:67-83)
+__device__ __forceinline__ void advance_clock(TimeState *ts, int add_dt, int add_step, int snap, double toutput_flow) {
+    if (add_dt) ts->t += ts->dt;
+    if (add_step) ts->step += 1.0;
+    if (snap && (ts->t - ts->t_lastsnap + 1e-8) >= toutput_flow) ts->t_lastsnap += toutput_flow;
+}
+
 __device__ __forceinline__ void kvec_at(const KGeom &g, int i, int j, int k, double &kx, double &ky,
                                         double &kz, double &m) {
     const int ii = i < g.nx / 2 ? i : i - g.nx;  // fmod(i + NX/2, NX) - NX/2
@@ -228,9 +236,11 @@ template <class T>
 __host__ __device__ constexpr int zmid_e(int m) {
     return line_e(m, 4);
 }
+// 256 threads a block; one wavefront for rows of NZ <= 64, so that small grids
+// spread over the CUs (64^3 HD FP64: 13.9 -> 12.4 us)
 template <class T>
 __host__ __device__ constexpr int zmid_rw(int m) {
-    return (m / zmid_e<T>(m)) >= 256 ? 1 : 256 / (m / zmid_e<T>(m));
+    return (m / zmid_e<T>(m)) >= 256 ? 1 : (m <= 32 ? 64 : 256) / (m / zmid_e<T>(m));
 }
 
 // BAT: a batched launch (blockIdx.z is the box); single-box launches use the
@@ -548,10 +558,16 @@ __global__ __launch_bounds__(256) void k_epilogue(const cpx<T> *__restrict__ P, 
 // tile autotune); TPL = N/EF threads per line, TCOLS columns per 256-thread block
 __host__ __device__ constexpr int fx_e(int n, int ef) { return line_e(n, ef); }
 __host__ __device__ constexpr int fx_tpl(int n, int ef) { return n / fx_e(n, ef); }
-// at most 64 columns: a lane past the last column repeats the last column's
-// loads and stores, which is safe only within the wave that owns that column
+// Threads of a block: 512 at 8 points per thread; at 4, which the autotune takes
+// where a grid has few columns, small blocks that spread them over the CUs (64^3
+// HD FP64, us per stage: 19.4 -> 14.9).  At most 64 columns: a lane past the last
+// column repeats the last column's loads and stores, which is safe only within
+// the wave that owns that column.
+__host__ __device__ constexpr int fx_threads(int n, int ef) { return ef == 8 ? 512 : (n <= 64 ? 128 : 256); }
 __host__ __device__ constexpr int fx_tcols(int n, int ef) {
-    return fx_tpl(n, ef) >= 512 ? 1 : (512 / fx_tpl(n, ef) < 64 ? 512 / fx_tpl(n, ef) : 64);
+    return fx_tpl(n, ef) >= fx_threads(n, ef)
+               ? 1
+               : (fx_threads(n, ef) / fx_tpl(n, ef) < 64 ? fx_threads(n, ef) / fx_tpl(n, ef) : 64);
 }
 
 // RK3 registers of the fused path.  Wray's scheme (hydro_mhd_advance.cu:114-164)
@@ -573,6 +589,8 @@ struct FusedConst {
     int inv;        // write the next stage's inverse x pass of the updated fields to W
     double scale;   // 1/(NX NY NZ) of the next inverse pass
     double cu, cs;  // coefficients of the stored increment in the current state and the base
+    int clock;      // stage 3: advance the step's clock (advance_clock)
+    double toutput_flow;
 };
 
 // Column tiles of the fused kernel: tile T holds the TC columns from T TC on of
@@ -1019,7 +1037,7 @@ __device__ __forceinline__ void fx_masked(const cpx<T> *__restrict__ probe, cpx<
 template <class T, int N, int LY, int MODE, int EF, bool STRAT = false>
 __global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilogue(
     const cpx<T> *P, const cpx<T> *__restrict__ probe, cpx<double> *__restrict__ U, cpx<T> *__restrict__ S,
-    cpx<T> *__restrict__ W, FusedConst fc, const cpx<T> *__restrict__ tw, const TimeState *__restrict__ ts, Batch bt) {
+    cpx<T> *__restrict__ W, FusedConst fc, const cpx<T> *__restrict__ tw, TimeState *ts, Batch bt) {
     using L = Layout<LY>;
     P = rebase(bt, 0, P);
     U = rebase(bt, 1, U);
@@ -1032,6 +1050,8 @@ __global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilog
         fc.e.nu_m = br->nu_m;
         fc.e.nu_th = br->nu_th;
     }
+    // the step ends here: every kernel of it reads dt alone of the clock
+    if (MODE == 3 && fc.clock && blockIdx.x + blockIdx.y + threadIdx.x == 0) advance_clock(ts, 1, 1, 1, fc.toutput_flow);
     constexpr int E = fx_e(N, EF);
     constexpr int TPL = N / E;
     constexpr int TC = fx_tcols(N, EF);

@@ -127,16 +127,13 @@ __global__ __launch_bounds__(256) void k_dt(const double *__restrict__ pmax, DtC
     ts->dt_sts = dt_sts;
 }
 
-// clock updates: t += dt (RungeKutta3), step++ (HydroMHDAdvance), snapshot
-// clock of CheckSnapshot (check_output.cu:67-83), tremap from the host
+// advance_clock, and tremap from the host
 __global__ void k_clock(TimeState *ts, int add_dt, int add_step, int snap, double toutput_flow,
                         int set_tremap, double tremap, Batch bt) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     ts = rebase(bt, 0, ts);
-    if (add_dt) ts->t += ts->dt;
-    if (add_step) ts->step += 1.0;
     if (set_tremap) ts->tremap = tremap;
-    if (snap && (ts->t - ts->t_lastsnap + 1e-8) >= toutput_flow) ts->t_lastsnap += toutput_flow;
+    advance_clock(ts, add_dt, add_step, snap, toutput_flow);
 }
 
 __global__ void k_set_time(TimeState *ts, double t, double step, double tls, double tremap) {
@@ -650,8 +647,7 @@ int launch_fwdx_rkl2(spk_ctx ctx, int bulk, int nx, const void *Q, void *U, void
                      const RklConst &c, int stage, double mu, double nu, double dtmut, double gdt, int inv,
                      double scale, const void *tw, const RklPlan *plan, const TimeState *ts, const void *probe);
 int launch_fwdx_epilogue(spk_ctx ctx, int bulk, int nx, int ly, int mode, int ef, const void *P, const void *probe,
-                         void *U, void *S, void *W, const FusedConst &fc, const void *tw, const TimeState *ts,
-                         int ngroups);
+                         void *U, void *S, void *W, const FusedConst &fc, const void *tw, TimeState *ts, int ngroups);
 bool plane_supported(const Grid3 &g, int prog);
 bool plane_rkl_supported(const Grid3 &g);
 int launch_plane(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int prog, const void *W, void *P,
@@ -996,6 +992,8 @@ int rhs_back_fused(spk_solver s, int mode, double gam, double xi, int project, i
     fc.e = make_epi(s, 0.0, gam, xi);
     fc.project = project;
     fc.inv = inv;
+    fc.clock = mode == 3;
+    fc.toutput_flow = s->p.toutput_flow;
     fc.scale = 1.0 / ((double)g.nx * g.ny * g.nz);
     // the increment register's coefficients (FusedConst): stage 2 forms U1 = U0 + g1 R0
     // and S1 = U0 + (g1 + x1) R0, stage 3 forms S2 = U2 + x2 R1
@@ -1454,8 +1452,7 @@ int step_fused(spk_solver s, bool w_valid) {
     SPK_TRY(rhs_front_from_w(s, false));
     SPK_TRY(rhs_back_fused(s, 2, gammaRK[1], xiRK[1], 0, 1));
     SPK_TRY(rhs_front_from_w(s, false));
-    SPK_TRY(rhs_back_fused(s, 3, gammaRK[2], 0.0, 1, 1));
-    SPK_TRY(clock(s, 1, 0, 0, 0, 0.0));
+    SPK_TRY(rhs_back_fused(s, 3, gammaRK[2], 0.0, 1, 1));  // and the step's clock
     s->fused_w_ok = true;
     if (sts && (s->step % 2) == 0) {
         SPK_TRY(cycle_from_w(2));  // W: stage 3's inverse x pass of the new state
@@ -1471,7 +1468,7 @@ int step_fused(spk_solver s, bool w_valid) {
     }
     s->step += 1;
     s->products_valid = false;
-    return clock(s, 0, 1, 0, 0, 0.0);
+    return SPK_OK;
 }
 
 void free_all(spk_solver s) {
@@ -1841,7 +1838,7 @@ int main_loop(spk_solver s, int nsteps, bool resume) {
                                                                           s->force_val, s->force_n, s->ts);
             SPK_LAUNCH_CHECK();
         }
-        SPK_TRY(clock(s, 0, 0, 1, 0, 0.0));
+        if (!fused) SPK_TRY(clock(s, 0, 0, 1, 0, 0.0));  // a fused step has done it
     }
     return SPK_OK;
 }
