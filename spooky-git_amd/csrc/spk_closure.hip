@@ -70,8 +70,28 @@ __device__ __forceinline__ float norm_cdf(float z) {
     const float e = 0.5f * erfc_pos(fabsf(z) * 0.70710678118654752f);
     return z > 0.0f ? 1.0f - e : e;
 }
-// GELU(z) = z Phi(z), GELU'(z) = Phi(z) + z phi(z)
-__device__ __forceinline__ float gelu(float z) { return z * norm_cdf(z); }
+// GELU(z) = z Phi(z) = max(z, 0) - |z| exp(-z^2 / 2) Q(t), t = 1 / (1 + 0.3 |z|):
+// Q is the minimax polynomial (relative error 5.7e-8 on |z| <= 13) of
+// exp(z^2 / 2) erfc(|z| / sqrt 2) / 2, fitted for this.  In FP32 against 64 bits
+// over |z| <= 12: largest error 2.4e-7, rms of the relative error for |z| < 4
+// 1.8e-7 (z norm_cdf(z): 3.8e-7 and 2.5e-7), in two thirds of the instructions.
+__device__ __forceinline__ float gelu(float z) {
+    const float a = fminf(fabsf(z), 16.0f);  // past it the tail is 0 in FP32
+    const float t = __builtin_amdgcn_rcpf(fmaf(a, 0.3f, 1.0f));
+    float q = 0.0382711252f;
+    q = fmaf(q, t, -0.168644095f);
+    q = fmaf(q, t, 0.227579084f);
+    q = fmaf(q, t, -0.0752666701f);
+    q = fmaf(q, t, 0.141676423f);
+    q = fmaf(q, t, 0.0950508391f);
+    q = fmaf(q, t, 0.12182595f);
+    q = fmaf(q, t, 0.119500989f);
+    q = fmaf(q, t, 6.38356403e-06f);
+    const float b = a * 0.84932180028801904f;  // sqrt(log2(e) / 2)
+    const float r = a * (__builtin_amdgcn_exp2f(-b * b) * q);
+    return z != z ? z : fmaxf(z, 0.0f) - r;
+}
+// GELU'(z) = Phi(z) + z phi(z)
 __device__ __forceinline__ float gelu_d(float z) {
     return norm_cdf(z) + z * 0.39894228040143268f * __expf(-0.5f * z * z);
 }
@@ -83,155 +103,264 @@ __device__ __forceinline__ int wrap(int i, int n) { return i < 0 ? i + n : (i >=
 // groups of 4 banks (64 banks of 4 bytes), and every tap's address is the lane's
 // base address plus a constant, so the transform needs no per-tap address registers.
 __host__ __device__ constexpr int xpitch(int cin) { return cin + 8; }
-constexpr size_t conv_lds(int cin) { return (size_t)(NTAP * CH * cin + HX * HY * HZ * xpitch(cin)) * sizeof(bf16); }
+constexpr size_t conv_lds(int cin) {
+    return (size_t)(NTAP * CH * cin + HX * HY * HZ * xpitch(cin)) * sizeof(bf16) + CH * sizeof(float);
+}
 
-constexpr int CONV_T = 512;  // 8 waves: two per SIMD, so one wave's LDS reads overlap the other's MFMAs
+constexpr int CONV_T = 512;  // 8 waves, two per SIMD
+
+// Bricks in the order that keeps halos in one XCD's L2: workgroups go to the 8
+// XCDs round robin, so workgroup w is on XCD w % 8 and takes bricks of that XCD's
+// eighth of the x range, x fastest, then z, then y: the bricks an XCD has at one
+// time share their halos, and only the eighth's own edges are read twice.
+struct Bricks {
+    int n, sx, x0, k, step, count;
+    __device__ Bricks(int n_) : n(n_) {
+        sx = n / 32;  // bricks along x in an eighth
+        x0 = (blockIdx.x & 7) * sx;
+        k = blockIdx.x >> 3;
+        step = gridDim.x >> 3;
+        count = (n / 4) * (n / 4) * (n / 32) / 8;
+    }
+    __device__ bool live() const { return k < count; }
+    __device__ bool more() const { return k + step < count; }
+    __device__ void origin(int kk, int &x, int &y, int &z) const {
+        const int r = kk / sx;
+        x = (x0 + kk - r * sx) * 4;
+        y = (r / sx) * 4;
+        z = (r % sx) * 32;
+    }
+};
 
 // One brick's input with its one-point halo (HX x HY x HZ points of CIN
-// channels, channels-last, periodic wrap), held in registers between its global
-// loads (fetch) and its LDS stores (stash: channels-last at the xpitch pitch;
-// stash_t: channel-major rows of the weight-gradient layout), so that a
-// block loads brick b + 1 while it computes brick b.
-template <int CIN>
+// channels, channels-last, periodic wrap), held in the registers of NT threads
+// between its global loads (fetch) and its LDS stores (stash), so that a block
+// loads the next brick while it computes one.  A chunk's place relative to the
+// brick's first point never changes: at[] keeps it, in 16-byte chunks, above
+// six bits that name the halo faces the chunk is on; a brick at a face of the grid
+// adds the wrap there.
+template <int CIN, int NT>
 struct HaloPrefetch {
     static constexpr int NQ = CIN / 8;
     static constexpr int NCH = HX * HY * HZ * NQ;  // 16-byte chunks
-    static constexpr int NPF = (NCH + CONV_T - 1) / CONV_T;
+    static constexpr int NPF = (NCH + NT - 1) / NT;
     bf16x8 v[NPF];
+    int at[NPF];
 
-    __device__ __forceinline__ void fetch(const bf16 *__restrict__ X, int b, int n, int tid) {
-        const int nbz = n / 32, nby = n / 4;
-        const int bz = b % nbz, by = (b / nbz) % nby, bx = b / (nbz * nby);
-        const int x0 = bx * 4, y0 = by * 4, z0 = bz * 32;
+    __device__ __forceinline__ HaloPrefetch(int n, int t) {
 #pragma unroll
         for (int k = 0; k < NPF; k++) {
-            const int i = tid + k * CONV_T;
-            if (i < NCH) {
-                const int q = i % NQ, hp = i / NQ;
-                const int hz = hp % HZ, hy = (hp / HZ) % HY, hx = hp / (HZ * HY);
-                const int gx = wrap(x0 + hx - 1, n), gy = wrap(y0 + hy - 1, n), gz = wrap(z0 + hz - 1, n);
-                v[k] = *reinterpret_cast<const bf16x8 *>(X + (((size_t)gx * n + gy) * n + gz) * CIN + 8 * q);
-            }
+            const int i = t + k * NT;
+            const int q = i % NQ, hp = i / NQ;
+            const int hz = hp % HZ, hy = (hp / HZ) % HY, hx = hp / (HZ * HY);
+            const int off = (((hx - 1) * n + hy - 1) * n + hz - 1) * NQ + q;
+            at[k] = off * 64 + (hx == 0) + 2 * (hx == HX - 1) + 4 * (hy == 0) + 8 * (hy == HY - 1) + 16 * (hz == 0) +
+                    32 * (hz == HZ - 1);
         }
     }
-    __device__ __forceinline__ void stash(bf16 *Xs, int tid) const {
+    __device__ __forceinline__ void fetch(const bf16 *__restrict__ X, const Bricks &br, int kk, int t) {
+        const int n = br.n;
+        int x0, y0, z0;
+        br.origin(kk, x0, y0, z0);
+        int o[NPF];
+#pragma unroll
+        for (int k = 0; k < NPF; k++) o[k] = at[k] >> 6;
+        auto wrap = [&](bool face, int bit, int by) {
+            if (face)
+#pragma unroll
+                for (int k = 0; k < NPF; k++) o[k] += (at[k] & bit) ? by : 0;
+        };
+        wrap(x0 == 0, 1, n * n * n * NQ);
+        wrap(x0 + 4 == n, 2, -n * n * n * NQ);
+        wrap(y0 == 0, 4, n * n * NQ);
+        wrap(y0 + 4 == n, 8, -n * n * NQ);
+        wrap(z0 == 0, 16, n * NQ);
+        wrap(z0 + 32 == n, 32, -n * NQ);
+        const bf16 *base = X + (((size_t)x0 * n + y0) * n + z0) * CIN;
+#pragma unroll
+        for (int k = 0; k < NPF; k++)
+            if (t + k * NT < NCH) v[k] = *reinterpret_cast<const bf16x8 *>(base + (ptrdiff_t)o[k] * 8);
+    }
+    __device__ __forceinline__ void stash(bf16 *Xs, int t, int pitch = xpitch(CIN)) const {
 #pragma unroll
         for (int k = 0; k < NPF; k++) {
-            const int i = tid + k * CONV_T;
-            if (i < NCH) {
-                const int q = i % NQ, hp = i / NQ;
-                *reinterpret_cast<bf16x8 *>(Xs + hp * xpitch(CIN) + 8 * q) = v[k];
-            }
+            const int i = t + k * NT;
+            if (i < NCH) *reinterpret_cast<bf16x8 *>(Xs + (i / NQ) * pitch + 8 * (i % NQ)) = v[k];
         }
     }
-    // Xs[ci][XPL]: halo point (hx, hy, hz) at (hx HY + hy) 48 + 7 + hz
-    template <int XPLEN>
-    __device__ __forceinline__ void stash_t_impl(bf16 *Xs, int tid) const {
-#pragma unroll
-        for (int k = 0; k < NPF; k++) {
-            const int i = tid + k * CONV_T;
-            if (i < NCH) {
-                const int q = i % NQ, hp = i / NQ;
-                const int hz = hp % HZ, hy = (hp / HZ) % HY, hx = hp / (HZ * HY);
-                const int e = (hx * HY + hy) * 48 + 7 + hz;
-#pragma unroll
-                for (int j = 0; j < 8; j++) Xs[(8 * q + j) * XPLEN + e] = v[k][j];
-            }
-        }
-    }
-    __device__ __forceinline__ void stash_t(bf16 *Xs, int tid) const;
 };
+
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+// swaps a's lanes 32..63 with b's lanes 0..31
+__device__ __forceinline__ void swap_halves(unsigned &a, unsigned &b) {
+    const u32x2 r = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a, b, false, false));
+    a = r[0];
+    b = r[1];
+}
+// A lane holds 4 channels (8 (r / 4) + 4 half + 0..3) of each of a point's four
+// channel groups g; lanes li and li + 32 the two halves.  For 16-byte accesses to
+// channels-last memory the pair exchanges groups: lane li then has the whole
+// groups 0 and 1, lane li + 32 groups 2 and 3, 32 contiguous bytes each.
+__device__ __forceinline__ void store_point(bf16 *__restrict__ P, int half, const bf16x4 (&v)[4]) {
+    unsigned d[4][2];
+    __builtin_memcpy(d, v, 32);
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) swap_halves(d[g][k], d[g + 2][k]);
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+        *reinterpret_cast<u32x4 *>(P + 16 * half + 8 * g) = u32x4{d[g][0], d[g][1], d[g + 2][0], d[g + 2][1]};
+}
+__device__ __forceinline__ void load_point(const bf16 *__restrict__ P, int half, u32x4 (&raw)[2]) {
+#pragma unroll
+    for (int g = 0; g < 2; g++) raw[g] = *reinterpret_cast<const u32x4 *>(P + 16 * half + 8 * g);
+}
+__device__ __forceinline__ void spread_point(const u32x4 (&raw)[2], bf16x4 (&v)[4]) {
+    unsigned d[4][2];
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            unsigned a = raw[g][k], b = raw[g][k + 2];
+            swap_halves(a, b);
+            d[g][k] = a;
+            d[g + 2][k] = b;
+        }
+    __builtin_memcpy(v, d, 32);
+}
 
 // MODE 0: hidden layer, Y = GELU(conv + b); 1: also Z = conv + b (training);
 // 2: output layer, out[c][p] = conv + b for c < 6 (FP32, channel-major);
 // 3: input gradient, Y = conv(dZ, flipped transposed W) * GELU'(Zp)
 
+// What bounds it: per brick (512 points) the MFMAs, the LDS reads of their
+// operands and the activation's VALU work are of one size, and a wave does them
+// one after the other.  So the two waves of a SIMD take turns: waves 0-3 compute
+// even bricks, waves 4-7 odd ones, and while one four has the matrix cores the
+// other makes the activation and the stores of the brick it computed before.  A
+// wave holds the four y columns of one x plane and takes the taps in groups of
+// one (dx, dz) and one K-chunk: 6 input columns and 3 weight fragments feed 12
+// MFMAs, half the LDS reads of a tap at a time.  With the brick order and 32-byte
+// stores of a point, 128^3, 32 -> 32 channels: 165 -> 134 us, with the stored Z
+// 180 -> 143, input gradient 190 -> 148.  Inputs in flight and out alone (no matrix
+// work, no activation) take 77 us of that, the MFMAs 46.
 template <int CIN, int MODE>
 __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, const bf16 *__restrict__ W,
                                                  const float *__restrict__ bias, bf16 *__restrict__ Y,
-                                                 bf16 *__restrict__ Z, const bf16 *__restrict__ Zp,
-                                                 float *__restrict__ out, int n) {
+                                                 bf16 *__restrict__ Z, const bf16 *__restrict__ Zp, int n) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     bf16 *Ws = reinterpret_cast<bf16 *>(smem);  // [27][32][CIN], chunk-swizzled by co
     bf16 *Xs = Ws + NTAP * CH * CIN;            // [HX*HY*HZ][xpitch(CIN)]
-    constexpr int NQ = CIN / 8;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    float *Bs = reinterpret_cast<float *>(Xs + HX * HY * HZ * xpitch(CIN));  // [32]
+    constexpr int NQ = CIN / 8, NKC = CIN / 16, NG = 9 * NKC;
+    static_assert(MODE == 0 || MODE == 1 || MODE == 3, "hidden layers and the input gradient");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int xw = w & 3, four = w >> 2;
     const int li = lane & 31, half = lane >> 5;
-    const int xw = w & 3, yg = 2 * (w >> 2);  // the wave's x plane and first of its two y columns
 
     for (int i = tid; i < NTAP * CH * NQ; i += CONV_T) {
         const int q = i % NQ, row = i / NQ;
         const bf16x8 v = *reinterpret_cast<const bf16x8 *>(W + (size_t)row * CIN + 8 * q);
         *reinterpret_cast<bf16x8 *>(Ws + row * CIN + 8 * swz(q, row & 31, CIN)) = v;
     }
-    const int nbz = n / 32, nby = n / 4;
-    const int nb = (n / 4) * nby * nbz;
-    const size_t P = (size_t)n * n * n;
-    HaloPrefetch<CIN> hf;
-    if (blockIdx.x < nb) hf.fetch(X, blockIdx.x, n, tid);
-    for (int b = blockIdx.x; b < nb; b += gridDim.x) {
-        const int bz = b % nbz, by = (b / nbz) % nby, bx = b / (nbz * nby);
-        const int x0 = bx * 4, y0 = by * 4, z0 = bz * 32;
-        __syncthreads();
-        hf.stash(Xs, tid);
-        __syncthreads();
-        // the next brick's loads are in flight during this brick's matrix work (the
-        // scheduling barrier keeps them ahead of it)
-        if (b + (int)gridDim.x < nb) hf.fetch(X, b + gridDim.x, n, tid);
-        __builtin_amdgcn_sched_barrier(0);
-        f32x16 acc[2];
+    Bricks br(n);
+    if (MODE != 3 && tid < CH) Bs[tid] = bias[tid];
+
+    f32x16 acc[4];
+    // D[co][point]: lane holds point li of column ys, co = 8 (r / 4) + 4 half + r % 4
+    auto finish = [&](int kk) {
+        int x0, y0, z0;
+        br.origin(kk, x0, y0, z0);
+        const size_t p0 = ((size_t)(x0 + xw) * n + y0) * n + z0 + li;
+        u32x4 zraw[MODE == 3 ? 4 : 1][2];
+        if constexpr (MODE == 3)
 #pragma unroll
-        for (int ys = 0; ys < 2; ys++)
+            for (int ys = 0; ys < 4; ys++) load_point(Zp + (p0 + (size_t)ys * n) * CH, half, zraw[MODE == 3 ? ys : 0]);
+#pragma unroll
+        for (int ys = 0; ys < 4; ys++) {
+            const size_t o = (p0 + (size_t)ys * n) * CH;
+            bf16x4 y[4], zz[4];
+            if constexpr (MODE == 3) spread_point(zraw[MODE == 3 ? ys : 0], zz);
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if constexpr (MODE == 3) {
+                        y[g][j] = (bf16)(acc[ys][4 * g + j] * gelu_d((float)zz[g][j]));
+                    } else {
+                        const float zf = acc[ys][4 * g + j] + Bs[8 * g + 4 * half + j];
+                        zz[g][j] = (bf16)zf;
+                        y[g][j] = (bf16)gelu(zf);
+                    }
+                }
+            store_point(Y + o, half, y);
+            if constexpr (MODE == 1) store_point(Z + o, half, zz);
+        }
+    };
+    auto matrix = [&]() {
+#pragma unroll
+        for (int ys = 0; ys < 4; ys++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[ys][r] = 0.0f;
+        bf16x8 a[2][3], x[2][6];
+        auto operands = [&](int g) {
+            const int kc = g % NKC, dz = (g / NKC) % 3 - 1, dx = g / (3 * NKC) - 1;
+            const int q = 2 * kc + half;
 #pragma unroll
-        for (int t = 0; t < NTAP; t++) {
-            const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
-#pragma unroll
-            for (int kc = 0; kc < CIN / 16; kc++) {
-                const int q = 2 * kc + half;
-                const bf16x8 a = *reinterpret_cast<const bf16x8 *>(Ws + (t * CH + li) * CIN + 8 * swz(q, li, CIN));
-#pragma unroll
-                for (int ys = 0; ys < 2; ys++) {
-                    const int hp = ((xw + 1 + dx) * HY + (yg + ys + 1 + dy)) * HZ + li + 1 + dz;
-                    const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(Xs + hp * xpitch(CIN) + 8 * q);
-                    acc[ys] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bv, acc[ys], 0, 0, 0);
-                }
+            for (int dy = 0; dy < 3; dy++) {
+                const int t = 9 * (dx + 1) + 3 * dy + dz + 1;
+                a[g & 1][dy] = *reinterpret_cast<const bf16x8 *>(Ws + (t * CH + li) * CIN + 8 * swz(q, li, CIN));
             }
-        }
-        // D[co][point]: lane holds point li, co = 8 (r / 4) + 4 half + r % 4
 #pragma unroll
-        for (int ys = 0; ys < 2; ys++) {
-            const size_t p = ((size_t)(x0 + xw) * n + (y0 + yg + ys)) * n + z0 + li;
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const int c0 = 8 * g + 4 * half;
-                if (MODE == 2) {
-                    if (c0 < 6) {
-#pragma unroll
-                        for (int j = 0; j < 4; j++)
-                            if (c0 + j < 6) out[(size_t)(c0 + j) * P + p] = acc[ys][4 * g + j] + bias[c0 + j];
-                    }
-                } else if (MODE == 3) {
-                    const bf16x4 zp = *reinterpret_cast<const bf16x4 *>(Zp + p * CH + c0);
-                    bf16x4 y;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) y[j] = (bf16)(acc[ys][4 * g + j] * gelu_d((float)zp[j]));
-                    *reinterpret_cast<bf16x4 *>(Y + p * CH + c0) = y;
-                } else {
-                    bf16x4 y, zz;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const float zf = acc[ys][4 * g + j] + bias[c0 + j];
-                        zz[j] = (bf16)zf;
-                        y[j] = (bf16)gelu(zf);
-                    }
-                    *reinterpret_cast<bf16x4 *>(Y + p * CH + c0) = y;
-                    if (MODE == 1) *reinterpret_cast<bf16x4 *>(Z + p * CH + c0) = zz;
-                }
+            for (int yy = 0; yy < 6; yy++) {
+                const int hp = ((xw + 1 + dx) * HY + yy) * HZ + li + 1 + dz;
+                x[g & 1][yy] = *reinterpret_cast<const bf16x8 *>(Xs + hp * xpitch(CIN) + 8 * q);
             }
+        };
+        operands(0);
+#pragma unroll
+        for (int g = 0; g < NG; g++) {
+            // one group ahead and no further: more operands in flight would spill
+            if (g + 1 < NG) operands(g + 1);
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+                for (int ys = 0; ys < 4; ys++)
+                    acc[ys] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[g & 1][dy], x[g & 1][ys + dy], acc[ys], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+
+    // 16 channels: the four whose turn it is puts its brick into LDS while the other,
+    // whose turn is next, loads the next brick; 32 channels: every wave takes part
+    // in both (a four's whole brick would be 80 registers a lane beside the
+    // accumulators and spill)
+    constexpr bool SPLIT = CIN == 16;
+    const int ft = SPLIT ? tid & 255 : tid;
+    HaloPrefetch<CIN, SPLIT ? CONV_T / 2 : CONV_T> hf(n, ft);
+    if (br.live() && !(SPLIT && four == 1)) hf.fetch(X, br, br.k, ft);
+    int turn = 0, last = -1;
+    for (; br.live(); br.k += br.step, turn ^= 1) {
+        __syncthreads();
+        if (!SPLIT || four == turn) hf.stash(Xs, ft);
+        else if (br.more()) hf.fetch(X, br, br.k + br.step, ft);
+        __syncthreads();
+        if (!SPLIT && br.more()) {
+            // in flight during this brick's matrix work (the scheduling barrier keeps
+            // the loads ahead of it)
+            hf.fetch(X, br, br.k + br.step, ft);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (four == turn) {
+            matrix();
+        } else if (last >= 0) {
+            finish(last);
+        }
+        last = br.k;
     }
+    if (last >= 0 && four != turn) finish(last);
 }
 
 // Output layer (32 -> 6 channels) on the 16-row matrix instruction
@@ -241,8 +370,16 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr size_t OUT_LDS = (size_t)(NTAP * 16 * CH + HX * HY * HZ * xpitch(CH)) * sizeof(bf16);
 
+// T = float: out[6][P], for the loss; T = double: the stresses themselves, times
+// their scales, in the padded real layout [6][n][n][n + 2] (pads 0), so that no
+// second pass converts them.
+struct OutScale {
+    double s[6];
+};
+template <class T>
 __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X, const bf16 *__restrict__ W,
-                                                     const float *__restrict__ bias, float *__restrict__ out, int n) {
+                                                     const float *__restrict__ bias, T *__restrict__ out, int n,
+                                                     OutScale sc) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     bf16 *Ws = reinterpret_cast<bf16 *>(smem);  // [27][16][32], chunk-swizzled by co
     bf16 *Xs = Ws + NTAP * 16 * CH;             // [HX*HY*HZ][xpitch(32)]
@@ -256,18 +393,17 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
         const bf16x8 v = *reinterpret_cast<const bf16x8 *>(W + ((size_t)t * CH + co) * CH + 8 * qq);
         *reinterpret_cast<bf16x8 *>(Ws + row * CH + 8 * swz(qq, co, CH)) = v;
     }
-    const int nbz = n / 32, nby = n / 4;
-    const int nb = (n / 4) * nby * nbz;
+    Bricks br(n);
     const size_t P = (size_t)n * n * n;
-    HaloPrefetch<CH> hf;
-    if (blockIdx.x < nb) hf.fetch(X, blockIdx.x, n, tid);
-    for (int b = blockIdx.x; b < nb; b += gridDim.x) {
-        const int bz = b % nbz, by = (b / nbz) % nby, bx = b / (nbz * nby);
-        const int x0 = bx * 4, y0 = by * 4, z0 = bz * 32;
+    HaloPrefetch<CH, CONV_T> hf(n, tid);
+    if (br.live()) hf.fetch(X, br, br.k, tid);
+    for (; br.live(); br.k += br.step) {
+        int x0, y0, z0;
+        br.origin(br.k, x0, y0, z0);
         __syncthreads();
         hf.stash(Xs, tid);
         __syncthreads();
-        if (b + (int)gridDim.x < nb) hf.fetch(X, b + gridDim.x, n, tid);
+        if (br.more()) hf.fetch(X, br, br.k + br.step, tid);
         __builtin_amdgcn_sched_barrier(0);
         f32x4 acc[2][2];  // [column][16-point half]
 #pragma unroll
@@ -276,18 +412,30 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
             for (int h = 0; h < 2; h++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) acc[c][h][r] = 0.0f;
+        // taps in groups of one (dx, dz): 4 input columns and 3 weight fragments feed
+        // 12 MFMAs
 #pragma unroll
-        for (int t = 0; t < NTAP; t++) {
-            const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(Ws + (t * 16 + l16) * CH + 8 * swz(q, l16, CH));
+        for (int g = 0; g < 9; g++) {
+            const int dx = g / 3 - 1, dz = g % 3 - 1;
+            bf16x8 a[3], x[4][2];
 #pragma unroll
-            for (int c = 0; c < 2; c++)
+            for (int dy = 0; dy < 3; dy++)
+                a[dy] = *reinterpret_cast<const bf16x8 *>(
+                    Ws + ((9 * (dx + 1) + 3 * dy + dz + 1) * 16 + l16) * CH + 8 * swz(q, l16, CH));
+#pragma unroll
+            for (int yy = 0; yy < 4; yy++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const int hp = ((xw + 1 + dx) * HY + (yg + c + 1 + dy)) * HZ + 16 * h + l16 + 1 + dz;
-                    const bf16x8 bv = *reinterpret_cast<const bf16x8 *>(Xs + hp * xpitch(CH) + 8 * q);
-                    acc[c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bv, acc[c][h], 0, 0, 0);
+                    const int hp = ((xw + 1 + dx) * HY + yg + yy) * HZ + 16 * h + l16 + 1 + dz;
+                    x[yy][h] = *reinterpret_cast<const bf16x8 *>(Xs + hp * xpitch(CH) + 8 * q);
                 }
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+                        acc[c][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[dy], x[c + dy][h], acc[c][h], 0, 0, 0);
         }
         // D[co][point]: lane holds point l16 of its half, co = 4 q + r
         if (q < 2) {
@@ -295,54 +443,89 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
             for (int c = 0; c < 2; c++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
-                    const size_t p = ((size_t)(x0 + xw) * n + (y0 + yg + c)) * n + z0 + 16 * h + l16;
+                    constexpr bool PAD = sizeof(T) == 8;
+                    const int z = z0 + 16 * h + l16;
+                    const size_t row = (size_t)(x0 + xw) * n + (y0 + yg + c);
+                    const size_t p = row * (PAD ? n + 2 : n) + z, fs = PAD ? (size_t)n * n * (n + 2) : P;
 #pragma unroll
                     for (int r = 0; r < 4; r++) {
                         const int co = 4 * q + r;
-                        if (co < 6) out[(size_t)co * P + p] = acc[c][h][r] + bias[co];
+                        if (co < 6) {
+                            const float v = acc[c][h][r] + bias[co];
+                            if constexpr (PAD) {
+                                const double s = r == 0 ? (q ? sc.s[4] : sc.s[0]) : r == 1 ? (q ? sc.s[5] : sc.s[1]) : sc.s[r];
+                                out[co * fs + p] = (double)v * s;
+                                if (z == n - 1) out[co * fs + p + 1] = out[co * fs + p + 2] = 0.0;
+                            } else {
+                                out[co * fs + p] = v;
+                            }
+                        }
                     }
                 }
         }
     }
 }
 
-// weight gradient, per-block partial sums part[block][27][32 co][32 ci]
-constexpr int DZS = 512 + 8;                 // dZ^T row (one co): 512 brick points + pad (65 16-byte slots)
-constexpr int XPL = HX * HY * 48 + 8;        // X^T plane (one ci): z rows of 48 + pad (217 slots)
-constexpr size_t DW_LDS = (size_t)(CH * DZS + CH * XPL) * sizeof(bf16);
+// Weight gradient, per-block partial sums part[block][27][32 co][32 ci], and the
+// bias gradient's bpart[block][32 co].  Both operands contract over points, so a
+// lane needs 8 points of one channel, while memory and LDS are channels-last: the
+// bricks are staged as they come, in 16-byte rows of 64-byte points, and the
+// transposing LDS read (ds_read_b64_tr_b16: 16 lanes give 4 points x 16 channels
+// and receive one channel's 4 points each) makes the fragments; a point pitch of
+// 64 bytes puts the 4 points of 32 lanes on all 64 banks once.  A tap's z shift is
+// an address, and the bias gradient is a 28th tap whose input is 1.  Staged
+// channel-major by 2-byte stores, with the shifts made in registers, half of the
+// LDS time was bank conflicts: 290 -> 156 us at 128^3, 32 channels, no conflicts
+// left; the MFMAs take 48 us of that.
+constexpr size_t dw_lds(int cin) { return (size_t)(512 * CH + HX * HY * HZ * cin) * sizeof(bf16); }
 
-template <int CIN>
-__device__ __forceinline__ void HaloPrefetch<CIN>::stash_t(bf16 *Xs, int tid) const {
-    stash_t_impl<XPL>(Xs, tid);
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+// rows p, p + 1, p + 2, p + 3 (pitch elements apart) of the lane's 16 channels: see above
+__device__ __forceinline__ bf16x8 tr_points8(const bf16 *p, int pitch) {
+    typedef __attribute__((address_space(3))) s16x4 *lds_p;
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_p)p);
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_p)(p + 4 * pitch));
+    bf16x8 v;
+    __builtin_memcpy(&v, &lo, 8);
+    __builtin_memcpy((char *)&v + 8, &hi, 8);
+    return v;
 }
 
 template <int CIN>
 __global__ __launch_bounds__(CONV_T) void k_conv_dw(const bf16 *__restrict__ X, const bf16 *__restrict__ dZ,
                                                  float *__restrict__ part, float *__restrict__ bpart, int n) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    bf16 *Ds = reinterpret_cast<bf16 *>(smem);  // [32 co][DZS]: point (bx, by, z) at (bx 4 + by) 32 + z
-    bf16 *Xs = Ds + CH * DZS;                   // [32 ci][XPL]: (hx, hy, z0 - 8 + e) at (hx 6 + hy) 48 + e
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    bf16 *Ds = reinterpret_cast<bf16 *>(smem);  // [512 points][32 co]: point (bx 4 + by) 32 + z
+    bf16 *Xs = Ds + 512 * CH;                   // [HX HY HZ points][CIN]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, half = lane >> 5;
-    for (int i = tid; i < CH * XPL; i += CONV_T) Xs[i] = (bf16)0.0f;  // padding and channels >= CIN stay 0
+    // the lane's part of a transposing read: point 8 half + (lane / 4) % 4 of 16, and
+    // 4 channels of its 16 (with 16 input channels the upper ones are 0)
+    const int rp = 8 * half + ((lane >> 2) & 3), chg = (lane >> 4) & 1, c4 = 4 * (lane & 3);
+    const bf16 *pa = Ds + rp * CH + 16 * chg + c4;
+    const bf16 *pb = Xs + rp * CIN + (CIN == 32 ? 16 * chg : 0) + c4;
     f32x16 acc[4];  // taps w, w + 8, w + 16, w + 24 of wave w
 #pragma unroll
     for (int k = 0; k < 4; k++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[k][r] = 0.0f;
-    // bias gradient: the block's sum of dZ per output channel, read from the
-    // bricks already in LDS; thread tid sums channel tid / 16, 8-point chunks
-    // (tid % 16) + 16 r of each brick (consecutive lanes, consecutive 16 bytes)
-    const int bco = tid >> 4, bseg = tid & 15;
-    float bacc = 0.0f;
-    const int nbz = n / 32, nby = n / 4;
-    const int nb = (n / 4) * nby * nbz;
-    HaloPrefetch<CIN> hf;
+    int toff[4];  // a tap's shift in the halo, elements
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int t = w + 8 * k;
+        toff[k] = (((t / 9) * HY + (t / 3) % 3) * HZ + t % 3) * CIN;
+    }
+    bf16x8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; j++) ones[j] = (bf16)1.0f;
+    Bricks br(n);
+    HaloPrefetch<CIN, CONV_T> hf(n, tid);
     constexpr int NPD = 512 * 4 / CONV_T;  // dZ chunks of 8 channels per thread
     bf16x8 pd[NPD];
-    auto fetch_dz = [&](int b) {
-        const int bz = b % nbz, by = (b / nbz) % nby, bx = b / (nbz * nby);
-        const int x0 = bx * 4, y0 = by * 4, z0 = bz * 32;
+    auto fetch_dz = [&](int kk) {
+        int x0, y0, z0;
+        br.origin(kk, x0, y0, z0);
 #pragma unroll
         for (int k = 0; k < NPD; k++) {
             const int i = tid + k * CONV_T;
@@ -351,79 +534,52 @@ __global__ __launch_bounds__(CONV_T) void k_conv_dw(const bf16 *__restrict__ X, 
             pd[k] = *reinterpret_cast<const bf16x8 *>(dZ + p * CH + 8 * q);
         }
     };
-    if (blockIdx.x < nb) {
-        fetch_dz(blockIdx.x);
-        hf.fetch(X, blockIdx.x, n, tid);
+    if (br.live()) {
+        fetch_dz(br.k);
+        hf.fetch(X, br, br.k, tid);
     }
-    for (int b = blockIdx.x; b < nb; b += gridDim.x) {
+    for (; br.live(); br.k += br.step) {
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < NPD; k++) {
-            const int i = tid + k * CONV_T;
-            const int q = i & 3, pt = i >> 2;
-#pragma unroll
-            for (int j = 0; j < 8; j++) Ds[(8 * q + j) * DZS + pt] = pd[k][j];
-        }
-        hf.stash_t(Xs, tid);
+        for (int k = 0; k < NPD; k++) *reinterpret_cast<bf16x8 *>(Ds + 8 * (tid + k * CONV_T)) = pd[k];
+        hf.stash(Xs, tid, CIN);
         __syncthreads();
         // the next brick's loads are in flight during this brick's matrix work
-        if (b + (int)gridDim.x < nb) {
-            fetch_dz(b + gridDim.x);
-            hf.fetch(X, b + gridDim.x, n, tid);
+        if (br.more()) {
+            fetch_dz(br.k + br.step);
+            hf.fetch(X, br, br.k + br.step, tid);
         }
         __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const bf16x8 v = *reinterpret_cast<const bf16x8 *>(Ds + bco * DZS + (bseg + 16 * r) * 8);
-#pragma unroll
-            for (int j = 0; j < 8; j++) bacc += (float)v[j];
-        }
+#pragma unroll 4
         for (int s = 0; s < 32; s++) {
-            const int run = 2 * s + half, col = run >> 2, zr = (run & 3) * 8;
-            const int bxl = col >> 2, byl = col & 3;
-            const bf16x8 a = *reinterpret_cast<const bf16x8 *>(Ds + li * DZS + col * 32 + zr);
+            const int col = s >> 1, zr = 16 * (s & 1);
+            const bf16x8 a = tr_points8(pa + (col * 32 + zr) * CH, CH);
+            const bf16 *xb = pb + (((col >> 2) * HY + (col & 3)) * HZ + zr) * CIN;
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int t = w + 8 * k;
-                if (t < NTAP) {
-                    const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
-                    const int base = li * XPL + ((bxl + 1 + dx) * HY + (byl + 1 + dy)) * 48 + 8 + zr;
-                    const u32x4 d = *reinterpret_cast<const u32x4 *>(Xs + base);
-                    u32x4 sv = d;
-                    if (dz > 0) {
-                        const unsigned ex = *reinterpret_cast<const unsigned *>(Xs + base + 8);
-                        sv[0] = __builtin_amdgcn_alignbit(d[1], d[0], 16);
-                        sv[1] = __builtin_amdgcn_alignbit(d[2], d[1], 16);
-                        sv[2] = __builtin_amdgcn_alignbit(d[3], d[2], 16);
-                        sv[3] = __builtin_amdgcn_alignbit(ex, d[3], 16);
-                    } else if (dz < 0) {
-                        const unsigned ex = *reinterpret_cast<const unsigned *>(Xs + base - 2);
-                        sv[0] = __builtin_amdgcn_alignbit(d[0], ex, 16);
-                        sv[1] = __builtin_amdgcn_alignbit(d[1], d[0], 16);
-                        sv[2] = __builtin_amdgcn_alignbit(d[2], d[1], 16);
-                        sv[3] = __builtin_amdgcn_alignbit(d[3], d[2], 16);
+                if (k < 3 || t < NTAP) {
+                    bf16x8 b = tr_points8(xb + toff[k], CIN);
+                    if constexpr (CIN == 16) {
+                        if (chg) b = bf16x8{};
                     }
-                    bf16x8 bv;
-                    __builtin_memcpy(&bv, &sv, 16);
-                    acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bv, acc[k], 0, 0, 0);
+                    acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[k], 0, 0, 0);
+                } else if (t == NTAP) {
+                    acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, ones, acc[k], 0, 0, 0);
                 }
             }
         }
     }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) bacc += __shfl_xor(bacc, o, 64);
-    if (bseg == 0) bpart[(size_t)blockIdx.x * CH + bco] = bacc;
     // D[co][ci]: lane holds ci = li, co = 8 (r / 4) + 4 half + r % 4
-    float *pb = part + (size_t)blockIdx.x * NTAP * CH * CH;
+    float *pb_ = part + (size_t)blockIdx.x * NTAP * CH * CH;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int t = w + 8 * k;
-        if (t < NTAP) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int co = 8 * (r / 4) + 4 * half + (r & 3);
-                pb[((size_t)t * CH + co) * CH + li] = acc[k][r];
-            }
+        for (int r = 0; r < 16; r++) {
+            const int co = 8 * (r / 4) + 4 * half + (r & 3);
+            if (t < NTAP) pb_[((size_t)t * CH + co) * CH + li] = acc[k][r];
+            else if (t == NTAP && li == 0) bpart[(size_t)blockIdx.x * CH + co] = acc[k][r];
         }
     }
 }
@@ -462,55 +618,34 @@ __global__ void k_pack_input(const double *__restrict__ u, bf16 *__restrict__ xi
     }
 }
 
-// normalized FP32 [6][P] <-> padded real FP64 [6][n][n][n + 2] with per-component scales
-__global__ void k_unpack_output(const float *__restrict__ out, double *__restrict__ tau, int n, double s0, double s1,
-                                double s2, double s3, double s4, double s5) {
-    const size_t P = (size_t)n * n * n;
-    const size_t fs = (size_t)n * n * (n + 2);
-    const double sc[6] = {s0, s1, s2, s3, s4, s5};
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 6 * fs; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i / fs);
-        const size_t e = i - (size_t)c * fs;
-        const size_t r = e / (n + 2), z = e - r * (n + 2);
-        tau[i] = z < (size_t)n ? (double)out[(size_t)c * P + r * n + z] * sc[c] : 0.0;
-    }
-}
-__global__ void k_prep_target(const double *__restrict__ tau, float *__restrict__ tgt, int n, double s0, double s1,
-                              double s2, double s3, double s4, double s5) {
-    const size_t P = (size_t)n * n * n;
-    const size_t fs = (size_t)n * n * (n + 2);
-    const double sc[6] = {s0, s1, s2, s3, s4, s5};
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < 6 * P; i += (size_t)gridDim.x * blockDim.x) {
-        const int c = (int)(i / P);
-        const size_t p = i - (size_t)c * P;
-        const size_t r = p / n, z = p - r * n;
-        tgt[i] = (float)(tau[(size_t)c * fs + r * (n + 2) + z] / sc[c]);
-    }
-}
-
-// loss = mean over 6 P of (pred - tgt)^2; dZ4[p][c] = 2 (pred - tgt) / (6 P) (c < 6, else 0)
-__global__ __launch_bounds__(256) void k_loss(const float *__restrict__ pred, const float *__restrict__ tgt,
-                                              bf16 *__restrict__ dz, size_t P, float *__restrict__ part) {
-    __shared__ float sm[256];
+// loss = mean over 6 P of (pred - tgt)^2, tgt = tau / scale from the padded real
+// layout; dZ4[p][c] = 2 (pred - tgt) / (6 P) (c < 6, else 0)
+constexpr int LOSS_T = 1024;
+__global__ __launch_bounds__(LOSS_T) void k_loss(const float *__restrict__ pred, const double *__restrict__ tau,
+                                                 bf16 *__restrict__ dz, int n, OutScale sc, float *__restrict__ part) {
+    __shared__ float sm[LOSS_T];
     float acc = 0.0f;
+    const size_t P = (size_t)n * n * n, fs = (size_t)n * n * (n + 2);
     const float g = 2.0f / (6.0f * (float)P);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (size_t)gridDim.x * blockDim.x) {
-        bf16x8 v0, v1, v2, v3;
-        for (int j = 0; j < 8; j++) v0[j] = v1[j] = v2[j] = v3[j] = (bf16)0.0f;
+        const size_t o = p + 2 * (p / n);
+        bf16x8 v0, v1;
+        for (int j = 0; j < 8; j++) v0[j] = v1[j] = (bf16)0.0f;
+#pragma unroll
         for (int c = 0; c < 6; c++) {
-            const float d = pred[(size_t)c * P + p] - tgt[(size_t)c * P + p];
+            const float d = pred[(size_t)c * P + p] - (float)(tau[(size_t)c * fs + o] / sc.s[c]);
             acc += d * d;
             v0[c] = (bf16)(g * d);
         }
-        bf16 *o = dz + p * CH;
-        *reinterpret_cast<bf16x8 *>(o) = v0;
-        *reinterpret_cast<bf16x8 *>(o + 8) = v1;
-        *reinterpret_cast<bf16x8 *>(o + 16) = v2;
-        *reinterpret_cast<bf16x8 *>(o + 24) = v3;
+        bf16 *q = dz + p * CH;
+        *reinterpret_cast<bf16x8 *>(q) = v0;
+        *reinterpret_cast<bf16x8 *>(q + 8) = v1;
+        *reinterpret_cast<bf16x8 *>(q + 16) = v1;
+        *reinterpret_cast<bf16x8 *>(q + 24) = v1;
     }
     sm[threadIdx.x] = acc;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
+    for (int s = LOSS_T / 2; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s) sm[threadIdx.x] += sm[threadIdx.x + s];
         __syncthreads();
     }
@@ -655,7 +790,7 @@ struct spk_closure_s {
     float *prm = nullptr, *grd = nullptr, *am = nullptr, *av = nullptr;  // FP32 master, gradient, Adam moments
     bf16 *Wb[4] = {}, *WT[4] = {};
     bf16 *xin = nullptr, *Z[3] = {}, *A[3] = {}, *dzA = nullptr, *dzB = nullptr;
-    float *out = nullptr, *tgt = nullptr, *part = nullptr, *bpart = nullptr, *lpart = nullptr;
+    float *out = nullptr, *part = nullptr, *bpart = nullptr, *lpart = nullptr;
     int adam_t = 0;
     double *tau = nullptr;          // coupling: padded real stresses [6][n][n][n + 2], transformed in place
     spk_fft_plan plan6 = nullptr;   // FP64 n^3 transforms of 6 fields
@@ -689,7 +824,6 @@ int closure_alloc(spk_closure c) {
     SPK_TRY(al((void **)&c->dzA, c->P * CH * 2));
     SPK_TRY(al((void **)&c->dzB, c->P * CH * 2));
     SPK_TRY(al((void **)&c->out, c->P * 6 * 4));
-    SPK_TRY(al((void **)&c->tgt, c->P * 6 * 4));
     SPK_TRY(al((void **)&c->part, (size_t)NBLK * NTAP * CH * CH * 4));
     SPK_TRY(al((void **)&c->bpart, (size_t)NBLK * CH * 4));
     SPK_TRY(al((void **)&c->lpart, (size_t)NBLK * 4));
@@ -701,7 +835,7 @@ int closure_alloc(spk_closure c) {
 
 void closure_free(spk_closure c) {
     if (c->plan6) spk_fft_plan_destroy(c->plan6);
-    void *b[] = {c->prm, c->grd, c->am, c->av, c->xin, c->dzA, c->dzB, c->out, c->tgt, c->part, c->bpart, c->lpart,
+    void *b[] = {c->prm, c->grd, c->am, c->av, c->xin, c->dzA, c->dzB, c->out, c->part, c->bpart, c->lpart,
                  c->tau};
     for (void *p : b)
         if (p) (void)hipFree(p);
@@ -722,10 +856,11 @@ int set_lds_attributes() {
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv<16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(16)));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_out, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OUT_LDS));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_out<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OUT_LDS));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_out<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OUT_LDS));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 3>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_dw<16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)DW_LDS));
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_dw<32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)DW_LDS));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_dw<16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dw_lds(16)));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv_dw<32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dw_lds(32)));
     done = true;
     return SPK_OK;
 }
@@ -745,7 +880,15 @@ unsigned conv_grid(spk_closure c) {
     return (unsigned)(nb < NBLK ? nb : NBLK);
 }
 
-int forward(spk_closure c, const void *u, bool train) {
+OutScale out_scale_of(spk_closure c) {
+    OutScale s;
+    for (int i = 0; i < 6; i++) s.s[i] = c->out_scale[i];
+    return s;
+}
+
+// tau: the stresses (inference); nullptr: training, the normalized stresses into c->out
+int forward(spk_closure c, const void *u, double *tau) {
+    const bool train = tau == nullptr;
     hipStream_t st = c->ctx->stream;
     const unsigned gp = (unsigned)((c->P + 255) / 256 < 4096 ? (c->P + 255) / 256 : 4096);
     k_pack_input<<<gp, 256, 0, st>>>((const double *)u, c->xin, c->n, (float)c->in_scale);
@@ -753,15 +896,16 @@ int forward(spk_closure c, const void *u, bool train) {
     const float *b[4];
     for (int l = 0; l < 4; l++) b[l] = c->prm + param_offset(l) + w_count(l);
     if (train) {
-        k_conv<16, 1><<<g, CONV_T, conv_lds(16), st>>>(c->xin, c->Wb[0], b[0], c->A[0], c->Z[0], nullptr, nullptr, c->n);
-        k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], c->Z[1], nullptr, nullptr, c->n);
-        k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], c->Z[2], nullptr, nullptr, c->n);
+        k_conv<16, 1><<<g, CONV_T, conv_lds(16), st>>>(c->xin, c->Wb[0], b[0], c->A[0], c->Z[0], nullptr, c->n);
+        k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], c->Z[1], nullptr, c->n);
+        k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], c->Z[2], nullptr, c->n);
     } else {
-        k_conv<16, 0><<<g, CONV_T, conv_lds(16), st>>>(c->xin, c->Wb[0], b[0], c->A[0], nullptr, nullptr, nullptr, c->n);
-        k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], nullptr, nullptr, nullptr, c->n);
-        k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], nullptr, nullptr, nullptr, c->n);
+        k_conv<16, 0><<<g, CONV_T, conv_lds(16), st>>>(c->xin, c->Wb[0], b[0], c->A[0], nullptr, nullptr, c->n);
+        k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], nullptr, nullptr, c->n);
+        k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], nullptr, nullptr, c->n);
     }
-    k_conv_out<<<g, CONV_T, OUT_LDS, st>>>(c->A[2], c->Wb[3], b[3], c->out, c->n);
+    if (train) k_conv_out<float><<<g, CONV_T, OUT_LDS, st>>>(c->A[2], c->Wb[3], b[3], c->out, c->n, out_scale_of(c));
+    else k_conv_out<double><<<g, CONV_T, OUT_LDS, st>>>(c->A[2], c->Wb[3], b[3], tau, c->n, out_scale_of(c));
     SPK_LAUNCH_CHECK();
     return SPK_OK;
 }
@@ -770,8 +914,8 @@ int forward(spk_closure c, const void *u, bool train) {
 int layer_grads(spk_closure c, int l, const bf16 *X, const bf16 *dz) {
     hipStream_t st = c->ctx->stream;
     const unsigned g = conv_grid(c);
-    if (CIN_L[l] == 16) k_conv_dw<16><<<g, CONV_T, DW_LDS, st>>>(X, dz, c->part, c->bpart, c->n);
-    else k_conv_dw<32><<<g, CONV_T, DW_LDS, st>>>(X, dz, c->part, c->bpart, c->n);
+    if (CIN_L[l] == 16) k_conv_dw<16><<<g, CONV_T, dw_lds(CIN_L[l]), st>>>(X, dz, c->part, c->bpart, c->n);
+    else k_conv_dw<32><<<g, CONV_T, dw_lds(CIN_L[l]), st>>>(X, dz, c->part, c->bpart, c->n);
     const int cnt = NTAP * CH * CH;
     // the [27][32][32] sums land in grd for cin = 32; for cin = 16 take ci < 16
     float *gw = c->grd + param_offset(l);
@@ -859,29 +1003,23 @@ extern "C" int spk_closure_set_scales(spk_closure c, double in_scale, const doub
 
 extern "C" int spk_closure_forward(spk_closure c, const void *u, void *tau) {
     SPK_REQUIRE(c && u && tau, SPK_ERR_ARG, "spk_closure_forward: null argument");
-    SPK_TRY(forward(c, u, false));
-    const double *s = c->out_scale;
-    k_unpack_output<<<4096, 256, 0, c->ctx->stream>>>(c->out, (double *)tau, c->n, s[0], s[1], s[2], s[3], s[4], s[5]);
-    SPK_LAUNCH_CHECK();
-    return SPK_OK;
+    return forward(c, u, (double *)tau);
 }
 
 extern "C" int spk_closure_grads(spk_closure c, const void *u, const void *tau_true, double *loss) {
     SPK_REQUIRE(c && u && tau_true, SPK_ERR_ARG, "spk_closure_grads: null argument");
     hipStream_t st = c->ctx->stream;
-    SPK_TRY(forward(c, u, true));
-    const double *s = c->out_scale;
-    k_prep_target<<<4096, 256, 0, st>>>((const double *)tau_true, c->tgt, c->n, s[0], s[1], s[2], s[3], s[4], s[5]);
-    k_loss<<<NBLK, 256, 0, st>>>(c->out, c->tgt, c->dzA, c->P, c->lpart);
+    SPK_TRY(forward(c, u, nullptr));
+    k_loss<<<NBLK, LOSS_T, 0, st>>>(c->out, (const double *)tau_true, c->dzA, c->n, out_scale_of(c), c->lpart);
     SPK_LAUNCH_CHECK();
     const unsigned g = conv_grid(c);
     // layer 4, then back through layers 3, 2, 1
     SPK_TRY(layer_grads(c, 3, c->A[2], c->dzA));
-    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzA, c->WT[3], nullptr, c->dzB, nullptr, c->Z[2], nullptr, c->n);
+    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzA, c->WT[3], nullptr, c->dzB, nullptr, c->Z[2], c->n);
     SPK_TRY(layer_grads(c, 2, c->A[1], c->dzB));
-    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzB, c->WT[2], nullptr, c->dzA, nullptr, c->Z[1], nullptr, c->n);
+    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzB, c->WT[2], nullptr, c->dzA, nullptr, c->Z[1], c->n);
     SPK_TRY(layer_grads(c, 1, c->A[0], c->dzA));
-    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzA, c->WT[1], nullptr, c->dzB, nullptr, c->Z[0], nullptr, c->n);
+    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzA, c->WT[1], nullptr, c->dzB, nullptr, c->Z[0], c->n);
     SPK_TRY(layer_grads(c, 0, c->xin, c->dzB));
     SPK_LAUNCH_CHECK();
     if (loss) {
@@ -927,10 +1065,7 @@ extern "C" int spk_closure_apply(spk_closure c, spk_solver s) {
         SPK_TRY(spk_fft_plan_create(c->ctx, n, n, n, SPK_F64, 6, &c->plan6));
     }
     SPK_TRY(spk_complex2real(s));
-    SPK_TRY(forward(c, v.realbuf + (size_t)v.VX * fs, false));
-    const double *sc = c->out_scale;
-    k_unpack_output<<<4096, 256, 0, c->ctx->stream>>>(c->out, c->tau, n, sc[0], sc[1], sc[2], sc[3], sc[4], sc[5]);
-    SPK_LAUNCH_CHECK();
+    SPK_TRY(forward(c, v.realbuf + (size_t)v.VX * fs, c->tau));
     SPK_TRY(spk_fft_r2c(c->plan6, c->tau, c->tau));
     k_sgs_update<<<4096, 256, 0, c->ctx->stream>>>(v.U + (long long)v.VX * v.ntc,
                                                    reinterpret_cast<const cpx<double> *>(c->tau), v.ntc, v.kg, v.ts);
