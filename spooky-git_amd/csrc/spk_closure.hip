@@ -4,24 +4,22 @@
 // FP32 accumulation; forward, backward (input and weight gradients) and Adam
 // written here.
 //
-//   layer 1: 3 (padded to 16) -> 32 channels, 3^3 taps, GELU
+//   layer 1: 3 -> 32 channels, 3^3 taps, GELU
 //   layers 2, 3: 32 -> 32, GELU
-//   layer 4: 32 -> 6 (padded to 32), linear: the normalized stress
+//   layer 4: 32 -> 6 (padded to 16), linear: the normalized stress
 //            tau_xx, tau_xy, tau_xz, tau_yy, tau_yz, tau_zz
 // Activations are channels-last [point][channel] BF16, point = (x n + y) n + z.
 //
 // Convolution as a GEMM per 4x4x32 brick of points: D[co][point] +=
 // W[tap][co][ci-chunk] x X[point + tap][ci-chunk], 27 taps x (CIN / 16)
-// K-chunks of 16 channels.  A block (8 waves: wave w takes x plane w % 4 and
-// the two y columns 2 (w / 4), 2 (w / 4) + 1 of 32 z points) keeps all 27 taps'
-// weights in LDS for its lifetime and stages each brick's input with a
-// one-point halo; blocks loop over bricks.  16-byte LDS reads are
-// conflict-free: the weights through an XOR swizzle of their 8-channel chunks
-// by output channel, the halo at a padded point pitch.  The weight gradient
-// contracts over points instead:
-// dW[tap][co][ci] = sum_p dZ[p][co] X[p + tap][ci], with both operands staged
-// channel-major so that a lane's 8 K values are 8 consecutive z points; the
-// +-1 z shift of a tap is made with 16-bit funnel shifts of aligned loads.
+// K-chunks of 16 channels.  A block of 8 waves keeps all 27 taps' weights in LDS
+// for its lifetime and stages each brick's input with a one-point halo; blocks
+// loop over bricks.  16-byte LDS reads are conflict-free: the weights through an
+// XOR swizzle of their 8-channel chunks by output channel, the halo at a padded
+// point pitch.  The first layer's K runs over taps and its 3 (4) channels
+// together, 7 K-chunks instead of 27.  The weight gradient contracts over points
+// instead: dW[tap][co][ci] = sum_p dZ[p][co] X[p + tap][ci], its operands
+// transposed by the LDS reads.
 #include "spk_internal.hpp"
 #include "spk_kernels.hpp"
 
@@ -333,26 +331,17 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
         }
     };
 
-    // 16 channels: the four whose turn it is puts its brick into LDS while the other,
-    // whose turn is next, loads the next brick; 32 channels: every wave takes part
-    // in both (a four's whole brick would be 80 registers a lane beside the
-    // accumulators and spill)
-    constexpr bool SPLIT = CIN == 16;
-    const int ft = SPLIT ? tid & 255 : tid;
-    HaloPrefetch<CIN, SPLIT ? CONV_T / 2 : CONV_T> hf(n, ft);
-    if (br.live() && !(SPLIT && four == 1)) hf.fetch(X, br, br.k, ft);
+    HaloPrefetch<CIN, CONV_T> hf(n, tid);
+    if (br.live()) hf.fetch(X, br, br.k, tid);
     int turn = 0, last = -1;
     for (; br.live(); br.k += br.step, turn ^= 1) {
         __syncthreads();
-        if (!SPLIT || four == turn) hf.stash(Xs, ft);
-        else if (br.more()) hf.fetch(X, br, br.k + br.step, ft);
+        hf.stash(Xs, tid);
         __syncthreads();
-        if (!SPLIT && br.more()) {
-            // in flight during this brick's matrix work (the scheduling barrier keeps
-            // the loads ahead of it)
-            hf.fetch(X, br, br.k + br.step, ft);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        // the next brick's loads are in flight during this brick's matrix work (the
+        // scheduling barrier keeps them ahead of it)
+        if (br.more()) hf.fetch(X, br, br.k + br.step, tid);
+        __builtin_amdgcn_sched_barrier(0);
         if (four == turn) {
             matrix();
         } else if (last >= 0) {
@@ -361,6 +350,85 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
         last = br.k;
     }
     if (last >= 0 && four != turn) finish(last);
+}
+
+// First layer (3 channels, kept as 4): the contraction over (tap t, channel c) is
+// one K index 4 t + c of 108, padded to 112, so 7 MFMAs make a column that 27
+// K-chunks of 16 padded channels made before; a lane's 8 K values are two taps'
+// points, two 8-byte LDS reads.  The weights stay in registers (28 of them), a
+// brick's halo is 9.8 KB, and four blocks share a CU and overlap their loads,
+// MFMAs, activation and stores, which bound it: 128^3, 108 -> 71 us.
+constexpr int KIN = 7;  // K-chunks of 16
+template <int MODE>
+__global__ __launch_bounds__(256, 4) void k_conv_in(const bf16 *__restrict__ X, const bf16 *__restrict__ W,
+                                                    const float *__restrict__ bias, bf16 *__restrict__ Y,
+                                                    bf16 *__restrict__ Z, int n) {
+    __shared__ bf16x4 Xs[HX * HY * HZ];
+    __shared__ float Bs[CH];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int li = lane & 31, half = lane >> 5;
+    Bricks br(n);
+    int x0, y0, z0;
+    br.origin(br.k, x0, y0, z0);
+    for (int i = tid; i < HX * HY * HZ; i += 256) {
+        const int hz = i % HZ, hy = (i / HZ) % HY, hx = i / (HZ * HY);
+        const int gx = wrap(x0 + hx - 1, n), gy = wrap(y0 + hy - 1, n), gz = wrap(z0 + hz - 1, n);
+        Xs[i] = *reinterpret_cast<const bf16x4 *>(X + (((size_t)gx * n + gy) * n + gz) * 4);
+    }
+    if (tid < CH) Bs[tid] = bias[tid];
+    bf16x8 a[KIN];
+    int off[KIN][2];  // halo points of the lane's two taps (the 28th tap's weights are 0)
+#pragma unroll
+    for (int kc = 0; kc < KIN; kc++) {
+        a[kc] = *reinterpret_cast<const bf16x8 *>(W + (kc * CH + li) * 16 + 8 * half);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int t = 4 * kc + 2 * half + j, u = t < NTAP ? t : NTAP - 1;
+            off[kc][j] = ((w + u / 9) * HY + (u / 3) % 3) * HZ + u % 3 + li;
+        }
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int yp = 0; yp < 4; yp += 2) {
+        f32x16 acc[2];
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[c][r] = 0.0f;
+#pragma unroll
+        for (int kc = 0; kc < KIN; kc++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const bf16x4 lo = Xs[off[kc][0] + (yp + c) * HZ], hi = Xs[off[kc][1] + (yp + c) * HZ];
+                const bf16x8 b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kc], b, acc[c], 0, 0, 0);
+            }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const size_t o = (((size_t)(x0 + w) * n + y0 + yp + c) * n + z0 + li) * CH;
+            bf16x4 y[4], zz[4];
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float zf = acc[c][4 * g + j] + Bs[8 * g + 4 * half + j];
+                    zz[g][j] = (bf16)zf;
+                    y[g][j] = (bf16)gelu(zf);
+                }
+            store_point(Y + o, half, y);
+            if constexpr (MODE == 1) store_point(Z + o, half, zz);
+        }
+    }
+}
+
+// its weights Wi[7][32 co][16]: K = 16 kc + kk = 4 t + c
+__global__ void k_pack_in(const float *__restrict__ W, bf16 *__restrict__ Wi) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= KIN * CH * 16) return;
+    const int kk = k % 16, co = (k / 16) % CH, K = 16 * (k / (16 * CH)) + kk;
+    const int t = K / 4, c = K % 4;
+    Wi[k] = t < NTAP && c < 3 ? (bf16)W[(t * CH + co) * 16 + c] : (bf16)0.0f;
 }
 
 // Output layer (32 -> 6 channels) on the 16-row matrix instruction
@@ -372,7 +440,7 @@ constexpr size_t OUT_LDS = (size_t)(NTAP * 16 * CH + HX * HY * HZ * xpitch(CH)) 
 
 // T = float: out[6][P], for the loss; T = double: the stresses themselves, times
 // their scales, in the padded real layout [6][n][n][n + 2] (pads 0), so that no
-// second pass converts them.
+// second pass converts them (128^3: 134 + 45 us -> 126; float 126 -> 100).
 struct OutScale {
     double s[6];
 };
@@ -601,20 +669,27 @@ __global__ void k_sum_parts(const float *__restrict__ part, int nparts, int coun
     atomicAdd(&grad[k], s);
 }
 
-// padded real FP64 u [3][n][n][n + 2] -> BF16 [P][16] (channels 3..15 zero), times in_scale
-__global__ void k_pack_input(const double *__restrict__ u, bf16 *__restrict__ xin, int n, float in_scale) {
+// padded real FP64 u [3][n][n][n + 2] -> BF16 [P][4] (channel 3 zero) for the first
+// layer, and [P][16] (channels 3..15 zero) for its weight gradient; times in_scale
+__global__ void k_pack_input(const double *__restrict__ u, bf16 *__restrict__ xin4, bf16 *__restrict__ xin, int n,
+                             float in_scale) {
     const size_t P = (size_t)n * n * n;
     const size_t fs = (size_t)n * n * (n + 2);
     for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (size_t)gridDim.x * blockDim.x) {
-        const size_t r = p / n, z = p - r * n;
-        const size_t o = r * (n + 2) + z;
-        bf16x8 v0, v1;
-        for (int j = 0; j < 8; j++) v0[j] = v1[j] = (bf16)0.0f;
-        v0[0] = (bf16)((float)u[o] * in_scale);
-        v0[1] = (bf16)((float)u[fs + o] * in_scale);
-        v0[2] = (bf16)((float)u[2 * fs + o] * in_scale);
-        *reinterpret_cast<bf16x8 *>(xin + p * 16) = v0;
-        *reinterpret_cast<bf16x8 *>(xin + p * 16 + 8) = v1;
+        const size_t o = p + 2 * (p / n);
+        bf16x4 v;
+        v[0] = (bf16)((float)u[o] * in_scale);
+        v[1] = (bf16)((float)u[fs + o] * in_scale);
+        v[2] = (bf16)((float)u[2 * fs + o] * in_scale);
+        v[3] = (bf16)0.0f;
+        *reinterpret_cast<bf16x4 *>(xin4 + p * 4) = v;
+        if (xin) {
+            bf16x8 v0, v1;
+            for (int j = 0; j < 8; j++) v0[j] = v1[j] = (bf16)0.0f;
+            for (int j = 0; j < 3; j++) v0[j] = v[j];
+            *reinterpret_cast<bf16x8 *>(xin + p * 16) = v0;
+            *reinterpret_cast<bf16x8 *>(xin + p * 16 + 8) = v1;
+        }
     }
 }
 
@@ -789,7 +864,7 @@ struct spk_closure_s {
     double in_scale = 1.0, out_scale[6] = {1, 1, 1, 1, 1, 1};
     float *prm = nullptr, *grd = nullptr, *am = nullptr, *av = nullptr;  // FP32 master, gradient, Adam moments
     bf16 *Wb[4] = {}, *WT[4] = {};
-    bf16 *xin = nullptr, *Z[3] = {}, *A[3] = {}, *dzA = nullptr, *dzB = nullptr;
+    bf16 *xin = nullptr, *xin4 = nullptr, *Z[3] = {}, *A[3] = {}, *dzA = nullptr, *dzB = nullptr;
     float *out = nullptr, *part = nullptr, *bpart = nullptr, *lpart = nullptr;
     int adam_t = 0;
     double *tau = nullptr;          // coupling: padded real stresses [6][n][n][n + 2], transformed in place
@@ -813,10 +888,11 @@ int closure_alloc(spk_closure c) {
     SPK_TRY(al((void **)&c->am, NP * 4));
     SPK_TRY(al((void **)&c->av, NP * 4));
     for (int l = 0; l < 4; l++) {
-        SPK_TRY(al((void **)&c->Wb[l], w_count(l) * 2));
+        SPK_TRY(al((void **)&c->Wb[l], (l ? w_count(l) : (size_t)KIN * CH * 16) * 2));
         if (l > 0) SPK_TRY(al((void **)&c->WT[l], w_count(l) * 2));
     }
     SPK_TRY(al((void **)&c->xin, c->P * 16 * 2));
+    SPK_TRY(al((void **)&c->xin4, c->P * 4 * 2));
     for (int l = 0; l < 3; l++) {
         SPK_TRY(al((void **)&c->Z[l], c->P * CH * 2));
         SPK_TRY(al((void **)&c->A[l], c->P * CH * 2));
@@ -835,7 +911,7 @@ int closure_alloc(spk_closure c) {
 
 void closure_free(spk_closure c) {
     if (c->plan6) spk_fft_plan_destroy(c->plan6);
-    void *b[] = {c->prm, c->grd, c->am, c->av, c->xin, c->dzA, c->dzB, c->out, c->part, c->bpart, c->lpart,
+    void *b[] = {c->prm, c->grd, c->am, c->av, c->xin, c->xin4, c->dzA, c->dzB, c->out, c->part, c->bpart, c->lpart,
                  c->tau};
     for (void *p : b)
         if (p) (void)hipFree(p);
@@ -852,8 +928,6 @@ void closure_free(spk_closure c) {
 int set_lds_attributes() {
     static bool done = false;
     if (done) return SPK_OK;
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<16, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(16)));
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(16)));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv_out<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OUT_LDS));
@@ -866,7 +940,8 @@ int set_lds_attributes() {
 }
 
 int pack_weights(spk_closure c) {
-    for (int l = 0; l < 4; l++) {
+    k_pack_in<<<(KIN * CH * 16 + 255) / 256, 256, 0, c->ctx->stream>>>(c->prm, c->Wb[0]);
+    for (int l = 1; l < 4; l++) {
         const int cnt = (int)w_count(l);
         k_pack_weights<<<(cnt + 255) / 256, 256, 0, c->ctx->stream>>>(c->prm + param_offset(l), c->Wb[l], c->WT[l],
                                                                      CIN_L[l]);
@@ -891,16 +966,17 @@ int forward(spk_closure c, const void *u, double *tau) {
     const bool train = tau == nullptr;
     hipStream_t st = c->ctx->stream;
     const unsigned gp = (unsigned)((c->P + 255) / 256 < 4096 ? (c->P + 255) / 256 : 4096);
-    k_pack_input<<<gp, 256, 0, st>>>((const double *)u, c->xin, c->n, (float)c->in_scale);
+    k_pack_input<<<gp, 256, 0, st>>>((const double *)u, c->xin4, train ? c->xin : nullptr, c->n, (float)c->in_scale);
+    const unsigned gin = (unsigned)((c->n / 4) * (c->n / 4) * (c->n / 32));
     const unsigned g = conv_grid(c);
     const float *b[4];
     for (int l = 0; l < 4; l++) b[l] = c->prm + param_offset(l) + w_count(l);
     if (train) {
-        k_conv<16, 1><<<g, CONV_T, conv_lds(16), st>>>(c->xin, c->Wb[0], b[0], c->A[0], c->Z[0], nullptr, c->n);
+        k_conv_in<1><<<gin, 256, 0, st>>>(c->xin4, c->Wb[0], b[0], c->A[0], c->Z[0], c->n);
         k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], c->Z[1], nullptr, c->n);
         k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], c->Z[2], nullptr, c->n);
     } else {
-        k_conv<16, 0><<<g, CONV_T, conv_lds(16), st>>>(c->xin, c->Wb[0], b[0], c->A[0], nullptr, nullptr, c->n);
+        k_conv_in<0><<<gin, 256, 0, st>>>(c->xin4, c->Wb[0], b[0], c->A[0], nullptr, c->n);
         k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], nullptr, nullptr, c->n);
         k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], nullptr, nullptr, c->n);
     }
