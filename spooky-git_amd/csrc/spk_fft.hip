@@ -385,6 +385,25 @@ int launch_pass_z_c2r(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int tin, 
     return tw.prec == SPK_F64 ? launch_z<double>(ctx, g, tw, false, a) : launch_z<float>(ctx, g, tw, false, a);
 }
 
+int launch_r2c(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const PassArgs &a) {
+    const PassArgs b{a.out, a.out, a.nfields, a.fstride_out, a.fstride_out, 1.0};
+    if (plane_yz_supported(g, tw.prec)) {
+        SPK_TRY(launch_plane_yz(ctx, g, tw, -1, a));
+    } else {
+        SPK_TRY(launch_pass_z_r2c(ctx, g, tw, tw.prec, tw.prec, a));
+        SPK_TRY(launch_pass_y(ctx, g, tw, -1, tw.prec, tw.prec, b));
+    }
+    return launch_pass_x(ctx, g, tw, -1, tw.prec, tw.prec, b);
+}
+
+int launch_c2r(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const PassArgs &a) {
+    const PassArgs b{a.out, a.out, a.nfields, a.fstride_out, a.fstride_out, 1.0};
+    SPK_TRY(launch_pass_x(ctx, g, tw, +1, tw.prec, tw.prec, a));
+    if (plane_yz_supported(g, tw.prec)) return launch_plane_yz(ctx, g, tw, +1, b);
+    SPK_TRY(launch_pass_y(ctx, g, tw, +1, tw.prec, tw.prec, b));
+    return launch_pass_z_c2r(ctx, g, tw, tw.prec, tw.prec, b);
+}
+
 }  // namespace spk
 
 // ------------------------------------------------------------------------
@@ -436,24 +455,16 @@ extern "C" int spk_fft_plan_destroy(spk_fft_plan p) {
 extern "C" int spk_fft_r2c(spk_fft_plan p, const void *in, void *out) {
     using namespace spk;
     SPK_REQUIRE(p && in && out, SPK_ERR_ARG, "spk_fft_r2c: null argument");
-    PassArgs a{in, out, p->batch, p->g.ntc, p->g.ntc, 1.0};
-    SPK_TRY(launch_pass_z_r2c(p->ctx, p->g, p->tw, p->prec, p->prec, a));
-    PassArgs b{out, out, p->batch, p->g.ntc, p->g.ntc, 1.0};
-    SPK_TRY(launch_pass_y(p->ctx, p->g, p->tw, -1, p->prec, p->prec, b));
-    SPK_TRY(launch_pass_x(p->ctx, p->g, p->tw, -1, p->prec, p->prec, b));
-    return SPK_OK;
+    const PassArgs a{in, out, p->batch, p->g.ntc, p->g.ntc, 1.0};
+    return launch_r2c(p->ctx, p->g, p->tw, a);
 }
 
 extern "C" int spk_fft_c2r(spk_fft_plan p, const void *in, void *out) {
     using namespace spk;
     SPK_REQUIRE(p && in && out, SPK_ERR_ARG, "spk_fft_c2r: null argument");
     const double scale = 1.0 / ((double)p->g.nx * p->g.ny * p->g.nz);
-    PassArgs a{in, out, p->batch, p->g.ntc, p->g.ntc, scale};
-    SPK_TRY(launch_pass_x(p->ctx, p->g, p->tw, +1, p->prec, p->prec, a));
-    PassArgs b{out, out, p->batch, p->g.ntc, p->g.ntc, 1.0};
-    SPK_TRY(launch_pass_y(p->ctx, p->g, p->tw, +1, p->prec, p->prec, b));
-    SPK_TRY(launch_pass_z_c2r(p->ctx, p->g, p->tw, p->prec, p->prec, b));
-    return SPK_OK;
+    const PassArgs a{in, out, p->batch, p->g.ntc, p->g.ntc, scale};
+    return launch_c2r(p->ctx, p->g, p->tw, a);
 }
 
 extern "C" int spk_fft_pass(spk_fft_plan p, int axis, int dir, const void *in, void *out) {

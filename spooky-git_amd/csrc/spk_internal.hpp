@@ -146,6 +146,14 @@ int launch_pass_z_r2c(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int tin, 
 int launch_pass_z_c2r(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int tin, int tout,
                       const PassArgs &a);
 
+// the y and z passes of a transform as one kernel, dir -1: real rows -> z R2C -> y,
+// +1: y -> z C2R -> real rows; in == out allowed (spk_planefft.hip)
+bool plane_yz_supported(const Grid3 &g, int prec);
+int launch_plane_yz(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, int dir, const PassArgs &a);
+// the whole transform of a.nfields fields: R2C, and C2R with the input scaled
+int launch_r2c(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const PassArgs &a);
+int launch_c2r(spk_ctx ctx, const Grid3 &g, const Twiddles &tw, const PassArgs &a);
+
 // looks up, with `device` current, the address of that device's copy of the
 // static scratch array behind spk_energy_noalloc (spk_solver.hip); once per device
 int noalloc_setup(int device);

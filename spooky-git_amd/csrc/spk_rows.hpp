@@ -111,6 +111,33 @@ struct ZRow {
         else FFTI::run(v, L, t, tw_m);
     }
 
+    // z values v (natural layout) -> the complex row in place, element k at L[PAD::at(k)],
+    // k = 0..M
+    __device__ static __forceinline__ void r2c_row(cpx<T> (&v)[E], cpx<T> *L, int t, const cpx<T> *__restrict__ tw_nz,
+                                                   const cpx<T> *__restrict__ tw_m) {
+        static_assert(!REG, "register twiddles: use r2c_tw");
+        FFTF::run(v, L, t, tw_m);
+#pragma unroll
+        for (int i = 0; i < E; i++) L[PAD::at(t + i * TPL)] = v[i];
+        lsync<WAVE>();
+        const T h = (T)0.5;
+        cpx<T> x[E];
+        const cpx<T> z0 = L[PAD::at(0)];
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            const int k = t + i * TPL;
+            const cpx<T> zk = v[i], zm = L[PAD::at((M - k) & (M - 1))];
+            const cpx<T> ev = {h * (zk.x + zm.x), h * (zk.y - zm.y)};
+            const cpx<T> od = {h * (zk.y + zm.y), -h * (zk.x - zm.x)};
+            x[i] = ev + cmul(od, tw_nz[k]);
+        }
+        lsync<WAVE>();
+#pragma unroll
+        for (int i = 0; i < E; i++) L[PAD::at(t + i * TPL)] = x[i];
+        if (t == 0) L[PAD::at(M)] = cpx<T>{z0.x - z0.y, (T)0};
+        lsync<WAVE>();
+    }
+
     // z values v (natural layout) -> complex row dst[0..M].  Ends with a barrier
     // so the caller may reuse L immediately.
     template <class TO>

@@ -1802,11 +1802,8 @@ extern "C" int spk_clean_divergence(spk_solver s) {
 extern "C" int spk_complex2real(spk_solver s) {
     SPK_CHECK_SOLVER_RO(s);
     const Grid3 &g = s->g;
-    PassArgs a{s->U, s->realbuf, s->nf, g.ntc, g.ntc, 1.0 / ((double)g.nx * g.ny * g.nz)};
-    SPK_TRY(launch_pass_x(s->ctx, g, s->tw64, +1, SPK_F64, SPK_F64, a));
-    PassArgs b{s->realbuf, s->realbuf, s->nf, g.ntc, g.ntc, 1.0};
-    SPK_TRY(launch_pass_y(s->ctx, g, s->tw64, +1, SPK_F64, SPK_F64, b));
-    return launch_pass_z_c2r(s->ctx, g, s->tw64, SPK_F64, SPK_F64, b);
+    const PassArgs a{s->U, s->realbuf, s->nf, g.ntc, g.ntc, 1.0 / ((double)g.nx * g.ny * g.nz)};
+    return launch_c2r(s->ctx, g, s->tw64, a);
 }
 
 extern "C" int spk_compute_dt(spk_solver s) {
@@ -1987,21 +1984,15 @@ namespace {
 // FP64 3D inverse transform of n complex fields (1/N folded in) into padded real rows
 int diag_c2r(spk_solver s, const void *in, void *out, int n) {
     const Grid3 &g = s->g;
-    PassArgs a{in, out, n, g.ntc, g.ntc, 1.0 / ((double)g.nx * g.ny * g.nz)};
-    SPK_TRY(launch_pass_x(s->ctx, g, s->tw64, +1, SPK_F64, SPK_F64, a));
-    PassArgs b{out, out, n, g.ntc, g.ntc, 1.0};
-    SPK_TRY(launch_pass_y(s->ctx, g, s->tw64, +1, SPK_F64, SPK_F64, b));
-    return launch_pass_z_c2r(s->ctx, g, s->tw64, SPK_F64, SPK_F64, b);
+    const PassArgs a{in, out, n, g.ntc, g.ntc, 1.0 / ((double)g.nx * g.ny * g.nz)};
+    return launch_c2r(s->ctx, g, s->tw64, a);
 }
 
 // FP64 3D forward transform of n padded real fields into complex fields
 int diag_r2c(spk_solver s, const void *in, void *out, int n) {
     const Grid3 &g = s->g;
-    PassArgs a{in, out, n, g.ntc, g.ntc, 1.0};
-    SPK_TRY(launch_pass_z_r2c(s->ctx, g, s->tw64, SPK_F64, SPK_F64, a));
-    PassArgs b{out, out, n, g.ntc, g.ntc, 1.0};
-    SPK_TRY(launch_pass_y(s->ctx, g, s->tw64, -1, SPK_F64, SPK_F64, b));
-    return launch_pass_x(s->ctx, g, s->tw64, -1, SPK_F64, SPK_F64, b);
+    const PassArgs a{in, out, n, g.ntc, g.ntc, 1.0};
+    return launch_r2c(s->ctx, g, s->tw64, a);
 }
 
 // twoFieldCorrelation of padded real fields: sum over physical points / N, added to *acc
@@ -2633,11 +2624,8 @@ bool aligned16(const void *p) { return p != nullptr && ((uintptr_t)p & 15u) == 0
 
 int complex2real_into(spk_solver s, const void *in, double *out, int nf) {
     const Grid3 &g = s->g;
-    PassArgs a{in, out, nf, g.ntc, g.ntc, 1.0 / ((double)g.nx * g.ny * g.nz)};
-    SPK_TRY(launch_pass_x(s->ctx, g, s->tw64, +1, SPK_F64, SPK_F64, a));
-    PassArgs b{out, out, nf, g.ntc, g.ntc, 1.0};
-    SPK_TRY(launch_pass_y(s->ctx, g, s->tw64, +1, SPK_F64, SPK_F64, b));
-    return launch_pass_z_c2r(s->ctx, g, s->tw64, SPK_F64, SPK_F64, b);
+    const PassArgs a{in, out, nf, g.ntc, g.ntc, 1.0 / ((double)g.nx * g.ny * g.nz)};
+    return launch_c2r(s->ctx, g, s->tw64, a);
 }
 
 // transform buffers of the anisotropic flux, made at the first call that needs them
