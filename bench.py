@@ -162,7 +162,9 @@ KERNEL_NAMES = {
 def kernel_table(spk, ctx, state, n, prec, fused, reps=10):
     """Live per-kernel average launch time (HIP events, spk_kernel_timings) and
     algorithmic HBM bytes per launch for the MHD step (6 state fields, 8 products);
-    fused: the step runs the fused forward-x/epilogue kernel (autotune's choice)."""
+    fused: the step runs the fused forward-x/epilogue kernel (autotune's choice).
+    The products cross HBM as the modes that the 2/3 mask keeps: kc of the n/2+1
+    columns after the z pass, and the rows |k_y| < kc of those after the y pass."""
     sol = spk.Solver(ctx, prec, **mhd_params(n))
     sol.set_fields(state)
     sol.main_loop(1)
@@ -171,11 +173,17 @@ def kernel_table(spk, ctx, state, n, prec, fused, reps=10):
     s64 = n * n * (n // 2 + 1) * 16
     sb = s64 if prec == "f64" else s64 // 2
     nin, nout, nf = 6, 8, 6
-    algo = {"inv_x": nin * (s64 + sb), "inv_y": nin * 2 * sb, "zmid": (nin + nout) * sb, "fwd_y": nout * 2 * sb,
-            "fwd_x": nout * 2 * sb, "epilogue": nout * sb + 4 * nf * s64, "clean_div": 2 * nf * s64,
-            # stage 2: products in, U0 and the increment register in, U2 and the new increment out
-            # (the register holds the bulk precision), next inverse x pass out
-            "fwdx_epilogue": nout * sb + 2 * nf * s64 + 2 * nf * sb + nin * sb}
+    kc = n // 3 + 1
+    fz = kc / (n // 2 + 1)  # share of a product's modes after the z pass
+    fzy = fz * (2 * kc - 1) / n  # and after the y pass
+    algo = {"inv_x": nin * (s64 + sb), "inv_y": nin * 2 * sb, "zmid": (nin + nout * fz) * sb,
+            "fwd_y": nout * (fz + fzy) * sb, "fwd_x": nout * 2 * fzy * sb,
+            "epilogue": nout * fzy * sb + 4 * nf * s64, "clean_div": 2 * nf * s64,
+            # stage 2: products in; in the mask's columns U0 and the increment register in, U2 and the
+            # new increment out (the register holds the bulk precision), in the others U0 in; next
+            # inverse x pass out
+            "fwdx_epilogue": nout * fzy * sb + fzy * (2 * nf * s64 + 2 * nf * sb) + (1 - fzy) * nf * s64 + nin * sb}
+    algo = {k: int(v) for k, v in algo.items()}
     if fused:
         # fused pipeline: forward x + epilogue + projection + next inverse x in one kernel
         per_step = {"inv_y": 3, "zmid": 3, "fwd_y": 3, "fwdx_epilogue": 3}

@@ -41,8 +41,7 @@ constexpr int CH = 32;                   // hidden channels
 constexpr int NTAP = 27;
 constexpr int NBLK = 256;                // persistent blocks (one per CU)
 
-__host__ __device__ constexpr int swz_shift(int cin) { return cin == 32 ? 2 : 3; }
-__device__ __forceinline__ int swz(int q, int p, int cin) { return q ^ ((p >> swz_shift(cin)) & (cin / 8 - 1)); }
+__device__ __forceinline__ int swz(int q, int p) { return q ^ ((p >> 2) & (CH / 8 - 1)); }
 
 // erfc(x) for x >= 0 by the Chebyshev fit of Press, Teukolsky, Vetterling and
 // Flannery, Numerical Recipes (2nd ed., sec. 6.2, erfcc): fractional error below
@@ -261,7 +260,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
     for (int i = tid; i < NTAP * CH * NQ; i += CONV_T) {
         const int q = i % NQ, row = i / NQ;
         const bf16x8 v = *reinterpret_cast<const bf16x8 *>(W + (size_t)row * CIN + 8 * q);
-        *reinterpret_cast<bf16x8 *>(Ws + row * CIN + 8 * swz(q, row & 31, CIN)) = v;
+        *reinterpret_cast<bf16x8 *>(Ws + row * CIN + 8 * swz(q, row & 31)) = v;
     }
     Bricks br(n);
     if (MODE != 3 && tid < CH) Bs[tid] = bias[tid];
@@ -309,7 +308,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
 #pragma unroll
             for (int dy = 0; dy < 3; dy++) {
                 const int t = 9 * (dx + 1) + 3 * dy + dz + 1;
-                a[g & 1][dy] = *reinterpret_cast<const bf16x8 *>(Ws + (t * CH + li) * CIN + 8 * swz(q, li, CIN));
+                a[g & 1][dy] = *reinterpret_cast<const bf16x8 *>(Ws + (t * CH + li) * CIN + 8 * swz(q, li));
             }
 #pragma unroll
             for (int yy = 0; yy < 6; yy++) {
@@ -459,7 +458,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
         const int qq = i & 3, row = i >> 2;  // row = t * 16 + co
         const int t = row >> 4, co = row & 15;
         const bf16x8 v = *reinterpret_cast<const bf16x8 *>(W + ((size_t)t * CH + co) * CH + 8 * qq);
-        *reinterpret_cast<bf16x8 *>(Ws + row * CH + 8 * swz(qq, co, CH)) = v;
+        *reinterpret_cast<bf16x8 *>(Ws + row * CH + 8 * swz(qq, co)) = v;
     }
     Bricks br(n);
     const size_t P = (size_t)n * n * n;
@@ -489,7 +488,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
 #pragma unroll
             for (int dy = 0; dy < 3; dy++)
                 a[dy] = *reinterpret_cast<const bf16x8 *>(
-                    Ws + ((9 * (dx + 1) + 3 * dy + dz + 1) * 16 + l16) * CH + 8 * swz(q, l16, CH));
+                    Ws + ((9 * (dx + 1) + 3 * dy + dz + 1) * 16 + l16) * CH + 8 * swz(q, l16));
 #pragma unroll
             for (int yy = 0; yy < 4; yy++)
 #pragma unroll

@@ -392,7 +392,7 @@ __host__ __device__ constexpr int zpass_rw(int m) { return zpass_tpl(m) >= 256 ?
 // whatever k_x is, so the forward transforms make only the columns the mask
 // keeps: the z pass stores the first kc of NZ/2+1 modes of a row, the y pass
 // transforms those columns and stores the rows with |k_y| index <= jc, moved
-// together (mode j > jc sits in row j - nskip).  At 256^3 that is 85 of 129
+// together (mode j > jc sits in row j - nskip).  At 256^3 that is 86 of 129
 // columns and 171 of 256 rows: the forward y pass reads 0.66 and writes 0.44 of
 // the full spectrum and the x pass reads 0.44 of it (8 fields at 256^3 FP64:
 // y pass 409 -> 254 us, x pass 447 -> 193 us; the FP64 step 6.68 -> 5.97 ms,

@@ -555,7 +555,7 @@ __global__ __launch_bounds__(256) void k_epilogue(const cpx<T> *__restrict__ P, 
 // come from k_inv_x).
 // ------------------------------------------------------------------------
 // EF: points per thread of the x line (4 or 8, chosen per grid by the solver's
-// tile autotune); TPL = N/EF threads per line, TCOLS columns per 256-thread block
+// tile autotune); TPL = N/EF threads per line, TCOLS columns per block
 __host__ __device__ constexpr int fx_e(int n, int ef) { return line_e(n, ef); }
 __host__ __device__ constexpr int fx_tpl(int n, int ef) { return n / fx_e(n, ef); }
 // Threads of a block: 512 at 8 points per thread; at 4, which the autotune takes
@@ -596,7 +596,7 @@ struct FusedConst {
 // Column tiles of the fused kernel: tile T holds the TC columns from T TC on of
 // the flattened (k_y, k_z) index, so that its accesses to the state and to W
 // start on whole 128-byte lines (a tile list cut at the mask's edges instead,
-// 85 of 129 columns, ran 20% slower: 1449 against 1207 us at 256^3 FP64 stage
+// 86 of 129 columns, ran 20% slower: 1449 against 1207 us at 256^3 FP64 stage
 // 2).  A tile with no column in the mask (fx_masked_tile) transforms no
 // product; in the others a column without products reads the (k_y, k_z) = 0
 // column's and multiplies it by m = 0.

@@ -1278,7 +1278,7 @@ int rkl2_back_fused(spk_solver s, int stage, double mu, double nu, double dtmut,
 // after the kernel that makes them, so that the host reads them while the GPU
 // works on: on even steps the RK3 stages are queued in between, on odd steps the
 // part of the cycle's first stage that needs neither.  Read at the cycle instead,
-// the GPU waited 45-58 us for the host in every step (512x512x2: 604 -> 556 us).
+// the GPU waited 45-58 us for the host in every step (512x512x2: 604 -> 561 us).
 int post_dt(spk_solver s) {
     if (s->nsts == 0 || s->rkl_device || s->ctx->rows) return SPK_OK;
     SPK_HIP(hipMemcpyAsync(s->h_ts, s->ts, sizeof(TimeState), hipMemcpyDeviceToHost, s->ctx->stream));
