@@ -36,10 +36,15 @@ struct PlaneShape {
     // 8 points of the plane per thread within a wave and 8 waves: with twice the threads, and
     // so fewer workgroups on a CU, 512x64x64 FP64 took 76 instead of 66 us
     static constexpr int T0 = NY * M / 8, PF_T = T0 < 64 ? 64 : (T0 > 512 ? 512 : T0);
-    static constexpr int EZ = line_e(M, 8), TPLZ = M / EZ, RW = PF_T / TPLZ;
+    // 8 points per thread, and 16 where 8 would leave the line a last pass of radix 2: its extra
+    // twiddles cost accuracy (FP32 rel-L2 of 64x16x32 1.36e-7 against 1.33e-7, of 64x16x256 1.49e-7
+    // against 1.48e-7; the separate passes 1.33e-7 and 1.48e-7), at up to 20% of the time of
+    // NZ = 256 transforms (512x16x256 FP64 C2R 60 -> 69 us, the separate passes 85)
+    static constexpr bool tail2(int n) { return n == 2 || (n > 8 && tail2(n / 8)); }
+    static constexpr int EZ = tail2(M) ? 16 : 8, TPLZ = M / EZ, RW = PF_T / TPLZ;
     static constexpr int ey(int e) { return (NZH + PF_T / (NY / e) - 1) / (PF_T / (NY / e)); }  // rounds of columns
-    // 16 points per thread where that saves a round of columns
-    static constexpr int EY = NY >= 16 && ey(16) < ey(8) ? 16 : 8;
+    // 16 also where that saves a round of columns
+    static constexpr int EY = tail2(NY) || ey(16) < ey(8) ? 16 : 8;
     static constexpr int TPLY = NY / EY, TC = PF_T / TPLY;
     static constexpr int ROWS = NY + (RW > NY ? 1 : 0);  // a spare row for row groups past the plane
     static constexpr size_t bytes = (size_t)ROWS * LL * sizeof(cpx<T>);
