@@ -20,6 +20,7 @@
 // together, 7 K-chunks instead of 27.  The weight gradient contracts over points
 // instead: dW[tap][co][ci] = sum_p dZ[p][co] X[p + tap][ci], its operands
 // transposed by the LDS reads.
+#include "spk_halo.hpp"
 #include "spk_internal.hpp"
 #include "spk_kernels.hpp"
 
@@ -36,7 +37,6 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int HX = 6, HY = 6, HZ = 34;  // brick 4 x 4 x 32 with a one-point halo
 constexpr int CH = 32;                   // hidden channels
 constexpr int NTAP = 27;
 constexpr int NBLK = 256;                // persistent blocks (one per CU)
@@ -132,10 +132,8 @@ struct Bricks {
 // One brick's input with its one-point halo (HX x HY x HZ points of CIN
 // channels, channels-last, periodic wrap), held in the registers of NT threads
 // between its global loads (fetch) and its LDS stores (stash), so that a block
-// loads the next brick while it computes one.  A chunk's place relative to the
-// brick's first point never changes: at[] keeps it, in 16-byte chunks, above
-// six bits that name the halo faces the chunk is on; a brick at a face of the grid
-// adds the wrap there.
+// loads the next brick while it computes one.  The chunks' places in a brick
+// (halo_place) are kept between bricks.
 template <int CIN, int NT>
 struct HaloPrefetch {
     static constexpr int NQ = CIN / 8;
@@ -146,37 +144,16 @@ struct HaloPrefetch {
 
     __device__ __forceinline__ HaloPrefetch(int n, int t) {
 #pragma unroll
-        for (int k = 0; k < NPF; k++) {
-            const int i = t + k * NT;
-            const int q = i % NQ, hp = i / NQ;
-            const int hz = hp % HZ, hy = (hp / HZ) % HY, hx = hp / (HZ * HY);
-            const int off = (((hx - 1) * n + hy - 1) * n + hz - 1) * NQ + q;
-            at[k] = off * 64 + (hx == 0) + 2 * (hx == HX - 1) + 4 * (hy == 0) + 8 * (hy == HY - 1) + 16 * (hz == 0) +
-                    32 * (hz == HZ - 1);
-        }
+        for (int k = 0; k < NPF; k++) at[k] = halo_place(t + k * NT, n, NQ);
     }
     __device__ __forceinline__ void fetch(const bf16 *__restrict__ X, const Bricks &br, int kk, int t) {
-        const int n = br.n;
         int x0, y0, z0;
         br.origin(kk, x0, y0, z0);
-        int o[NPF];
-#pragma unroll
-        for (int k = 0; k < NPF; k++) o[k] = at[k] >> 6;
-        auto wrap = [&](bool face, int bit, int by) {
-            if (face)
-#pragma unroll
-                for (int k = 0; k < NPF; k++) o[k] += (at[k] & bit) ? by : 0;
-        };
-        wrap(x0 == 0, 1, n * n * n * NQ);
-        wrap(x0 + 4 == n, 2, -n * n * n * NQ);
-        wrap(y0 == 0, 4, n * n * NQ);
-        wrap(y0 + 4 == n, 8, -n * n * NQ);
-        wrap(z0 == 0, 16, n * NQ);
-        wrap(z0 + 32 == n, 32, -n * NQ);
-        const bf16 *base = X + (((size_t)x0 * n + y0) * n + z0) * CIN;
+        unsigned o[NPF];
+        halo_chunks(at, o, br.n, NQ, x0, y0, z0);
 #pragma unroll
         for (int k = 0; k < NPF; k++)
-            if (t + k * NT < NCH) v[k] = *reinterpret_cast<const bf16x8 *>(base + (ptrdiff_t)o[k] * 8);
+            if (t + k * NT < NCH) v[k] = *reinterpret_cast<const bf16x8 *>(X + (size_t)o[k] * 8);
     }
     __device__ __forceinline__ void stash(bf16 *Xs, int t, int pitch = xpitch(CIN)) const {
 #pragma unroll
