@@ -86,7 +86,7 @@ __device__ __forceinline__ float gelu(float z) {
     q = fmaf(q, t, 6.38356403e-06f);
     const float b = a * 0.84932180028801904f;  // sqrt(log2(e) / 2)
     const float r = a * (__builtin_amdgcn_exp2f(-b * b) * q);
-    return z != z ? z : fmaxf(z, 0.0f) - r;
+    return z > -__builtin_inff() ? fmaxf(z, 0.0f) - r : __builtin_nanf("");  // NaN for NaN and, as z Phi(z), for -inf
 }
 // GELU'(z) = Phi(z) + z phi(z)
 __device__ __forceinline__ float gelu_d(float z) {
