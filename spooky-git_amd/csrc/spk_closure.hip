@@ -354,7 +354,7 @@ __global__ __launch_bounds__(256, 4) void k_conv_in(const bf16 *__restrict__ X, 
     }
     if (tid < CH) Bs[tid] = bias[tid];
     bf16x8 a[KIN];
-    int off[KIN][2];  // halo points of the lane's two taps (the 28th tap's weights are 0)
+    int off[KIN][2];  // halo points of the lane's two taps (the 28th, past the end, reads as 0)
 #pragma unroll
     for (int kc = 0; kc < KIN; kc++) {
         a[kc] = *reinterpret_cast<const bf16x8 *>(W + (kc * CH + li) * 16 + 8 * half);
@@ -376,7 +376,9 @@ __global__ __launch_bounds__(256, 4) void k_conv_in(const bf16 *__restrict__ X, 
         for (int kc = 0; kc < KIN; kc++)
 #pragma unroll
             for (int c = 0; c < 2; c++) {
-                const bf16x4 lo = Xs[off[kc][0] + (yp + c) * HZ], hi = Xs[off[kc][1] + (yp + c) * HZ];
+                const bf16x4 lo = Xs[off[kc][0] + (yp + c) * HZ];
+                bf16x4 hi = Xs[off[kc][1] + (yp + c) * HZ];
+                if (4 * kc + 3 >= NTAP && half) hi = bf16x4{};  // its weights are 0 too, but 0 inf is NaN
                 const bf16x8 b = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
                 acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kc], b, acc[c], 0, 0, 0);
             }

@@ -44,3 +44,10 @@ def test_minus_infinity(at):
     tau, box = stresses(-np.inf, at), reach(at)
     assert np.all(np.isnan(tau[:, box]))
     assert np.all(np.isfinite(tau[:, ~box]))
+
+
+@pytest.mark.parametrize("at", AT)
+def test_plus_infinity(at):
+    tau, box = stresses(np.inf, at), reach(at)
+    assert np.all(np.isposinf(tau[:, box]))
+    assert np.all(np.isfinite(tau[:, ~box]))
