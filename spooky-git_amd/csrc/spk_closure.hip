@@ -565,6 +565,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv_dw(const bf16 *__restrict__ X, 
     bf16x8 ones;
 #pragma unroll
     for (int j = 0; j < 8; j++) ones[j] = (bf16)1.0f;
+    float bsum = 0.0f;  // bias gradient of co = li: the bricks' sums are added up apart from the 32 steps within one
     Bricks br(n);
     HaloPrefetch<CIN, CONV_T> hf(n, tid);
     constexpr int NPD = 512 * 4 / CONV_T;  // dZ chunks of 8 channels per thread
@@ -611,13 +612,19 @@ __global__ __launch_bounds__(CONV_T) void k_conv_dw(const bf16 *__restrict__ X, 
                     }
                     acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[k], 0, 0, 0);
                 } else if (t == NTAP) {
-                    acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, ones, acc[k], 0, 0, 0);
+                    acc[k] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ones, a, acc[k], 0, 0, 0);  // rows alike
                 }
             }
+        }
+        if (w + 24 == NTAP) {
+            bsum += acc[3][0];
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[3][r] = 0.0f;
         }
     }
     // D[co][ci]: lane holds ci = li, co = 8 (r / 4) + 4 half + r % 4
     float *pb_ = part + (size_t)blockIdx.x * NTAP * CH * CH;
+    if (w + 24 == NTAP && half == 0) bpart[(size_t)blockIdx.x * CH + li] = bsum;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int t = w + 8 * k;
@@ -625,7 +632,6 @@ __global__ __launch_bounds__(CONV_T) void k_conv_dw(const bf16 *__restrict__ X, 
         for (int r = 0; r < 16; r++) {
             const int co = 8 * (r / 4) + 4 * half + (r & 3);
             if (t < NTAP) pb_[((size_t)t * CH + co) * CH + li] = acc[k][r];
-            else if (t == NTAP && li == 0) bpart[(size_t)blockIdx.x * CH + co] = acc[k][r];
         }
     }
 }
