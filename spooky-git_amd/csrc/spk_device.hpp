@@ -103,14 +103,29 @@ __device__ __forceinline__ void dft4(cpx<T>& x0, cpx<T>& x1, cpx<T>& x2, cpx<T>&
     x3 = b - d;
 }
 
-template <int DIR, class T>
+// a exp(DIR 2 pi i / 8) with sqrt(1/2) to twice FP64's precision: its nearest double is
+// off by 0.61 of a unit roundoff (the nearest float by 0.29), in every product alike
+template <int DIR>
+__device__ __forceinline__ cpx<double> weighth(cpx<double> a) {
+    constexpr double hi = 0.70710678118654757, lo = -4.833646656726457e-17;
+    const double p = a.x - DIR * a.y, q = a.y + DIR * a.x;
+    return {fma(p, hi, p * lo), fma(q, hi, q * lo)};
+}
+
+// EXACT: sqrt(1/2) as in weighth
+template <int DIR, bool EXACT = false, class T>
 __device__ __forceinline__ void dft8(cpx<T> (&v)[8]) {
     // n = n1 + 2 n2 (n1<2, n2<4), k = k2 + 4 k1
     dft4<DIR>(v[0], v[2], v[4], v[6]);
     dft4<DIR>(v[1], v[3], v[5], v[7]);
-    v[3] = wconst<1, 8, DIR>(v[3]);
+    if constexpr (EXACT) {
+        v[3] = weighth<DIR>(v[3]);
+        v[7] = wconst<2, 8, DIR>(weighth<DIR>(v[7]));
+    } else {
+        v[3] = wconst<1, 8, DIR>(v[3]);
+        v[7] = wconst<3, 8, DIR>(v[7]);
+    }
     v[5] = wconst<2, 8, DIR>(v[5]);
-    v[7] = wconst<3, 8, DIR>(v[7]);
     cpx<T> o[8];
 #pragma unroll
     for (int k2 = 0; k2 < 4; k2++) {
@@ -149,7 +164,7 @@ __device__ __forceinline__ void dft16(cpx<T> (&v)[16]) {
 }
 
 // DFT of R values taken from v at indices OFF + r*STRIDE (compile-time), in place
-template <int R, int DIR, int OFF, int STRIDE, int E, class T>
+template <int R, int DIR, int OFF, int STRIDE, bool EXACT, int E, class T>
 __device__ __forceinline__ void dft_group(cpx<T> (&v)[E]) {
     if constexpr (R == 1) {
         return;
@@ -161,7 +176,7 @@ __device__ __forceinline__ void dft_group(cpx<T> (&v)[E]) {
         cpx<T> g[R];
 #pragma unroll
         for (int r = 0; r < R; r++) g[r] = v[OFF + r * STRIDE];
-        if constexpr (R == 8) dft8<DIR>(g);
+        if constexpr (R == 8) dft8<DIR, EXACT>(g);
         else dft16<DIR>(g);
 #pragma unroll
         for (int r = 0; r < R; r++) v[OFF + r * STRIDE] = g[r];
@@ -238,7 +253,8 @@ struct LineTw {
     cpx<T> wt[NW];
 };
 
-template <class T, int N, int E, int DIR, bool WAVE = false, int TWM = 0, class PAD = PadSkew>
+// EXACT (FP64): radix-8 butterflies by weighth.
+template <class T, int N, int E, int DIR, bool WAVE = false, int TWM = 0, class PAD = PadSkew, bool EXACT = false>
 struct LineFFT {
     static_assert(N % E == 0, "E must divide N");
     static constexpr int TPL = N / E;                  // threads per line
@@ -298,7 +314,7 @@ struct LineFFT {
                 v[r] = cmul(v[r], wr);
             }
         }
-        dft_group<E, DIR, 0, 1>(v);
+        dft_group<E, DIR, 0, 1, EXACT>(v);
         cpx<T> wn[NW];
         if constexpr (TWM == 1) {
             if constexpr (P + 1 < NPASS) {
@@ -338,7 +354,7 @@ struct LineFFT {
             else wr = tw_tail(t, M, r, tw);
             v[M + r * G] = cmul(v[M + r * G], wr);
         }
-        dft_group<B, DIR, M, G>(v);
+        dft_group<B, DIR, M, G, EXACT>(v);
         if constexpr (M + 1 < G) pass_tail<M + 1>(v, t, tw, w, tr);
     }
 

@@ -45,6 +45,11 @@ struct PlaneShape {
     static constexpr int ey(int e) { return (NZH + PF_T / (NY / e) - 1) / (PF_T / (NY / e)); }  // rounds of columns
     // 16 also where that saves a round of columns
     static constexpr int EY = tail2(NY) || ey(16) < ey(8) ? 16 : 8;
+    // FP64: two radix-8 passes with sqrt(1/2) rounded to FP64 were off by up to 2.8% more than the
+    // separate passes' radix 16 and 4 (rel-L2 of 32x16x128 2.54e-16 against 2.48e-16; with it to
+    // twice the precision 2.46e-16; NZ = 512 2.73e-16, 2.69e-16 and 2.64e-16), in the same time.  16 points
+    // there instead took 10-40% longer (512x16x512 C2R 104 -> 150 us)
+    static constexpr bool EXACT = sizeof(T) == 8;
     static constexpr int TPLY = NY / EY, TC = PF_T / TPLY;
     static constexpr int ROWS = NY + (RW > NY ? 1 : 0);  // a spare row for row groups past the plane
     static constexpr size_t bytes = (size_t)ROWS * LL * sizeof(cpx<T>);
@@ -56,7 +61,7 @@ __global__ __launch_bounds__((PlaneShape<T, NY, NZ>::PF_T)) void k_plane_yz(
     const cpx<T> *in, cpx<T> *out, long long fs_in, long long fs_out, const cpx<T> *__restrict__ twy,
     const cpx<T> *__restrict__ tw_nz, const cpx<T> *__restrict__ tw_m, Batch bt) {
     using S = PlaneShape<T, NY, NZ>;
-    using Row = ZRow<T, S::M, S::EZ>;
+    using Row = ZRow<T, S::M, S::EZ, false, S::EXACT>;
     constexpr int M = S::M, NZH = S::NZH, LL = S::LL;
     static_assert(Row::WAVE && Row::LL == LL, "a row's threads share one wavefront");
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -82,7 +87,7 @@ __global__ __launch_bounds__((PlaneShape<T, NY, NZ>::PF_T)) void k_plane_yz(
                 else v[i] = L[n * LL];
             }
             if constexpr (DIR < 0) __syncthreads();  // a line's values are read before its exchanges overwrite them
-            LineFFT<T, NY, S::EY, DIR, false, 0, PadColumn<LL>>::run(v, L, t, twy);
+            LineFFT<T, NY, S::EY, DIR, false, 0, PadColumn<LL>, S::EXACT>::run(v, L, t, twy);
 #pragma unroll
             for (int i = 0; i < S::EY; i++) {
                 const int n = t + i * S::TPLY;

@@ -19,15 +19,15 @@ namespace spk {
 // REG: the kernel loads a thread's twiddles once (load_tw) and hands them to
 // every transform of the row (c2r_regs / r2c with a RowTw); otherwise each
 // twiddle is read from the tables where it is used.
-template <class T, int M, int E, bool REG = false>
+template <class T, int M, int E, bool REG = false, bool EXACT = false>
 struct ZRow {
     static constexpr int TPL = M / E;
     using PAD = PadXor;
     static constexpr int LL = PAD::len(M + 1);  // LDS elements per row
     // the threads of a row share one wavefront: wavefront-level ordering only
     static constexpr bool WAVE = TPL <= 64;
-    using FFTI = LineFFT<T, M, E, +1, WAVE, REG ? 2 : 0, PAD>;
-    using FFTF = LineFFT<T, M, E, -1, WAVE, REG ? 2 : 0, PAD>;
+    using FFTI = LineFFT<T, M, E, +1, WAVE, REG ? 2 : 0, PAD, EXACT>;
+    using FFTF = LineFFT<T, M, E, -1, WAVE, REG ? 2 : 0, PAD, EXACT>;
 
     // a thread's twiddles: the length-M FFT's and W^k = exp(-2 pi i k / NZ) of
     // its points k = t + i*TPL for the split pre/post-processing
