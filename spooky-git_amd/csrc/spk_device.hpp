@@ -424,6 +424,13 @@ struct ProdLay {
 __host__ __device__ __forceinline__ int prod_row(const ProdLay &l, int j) {
     return j <= l.jc ? j : (j > l.jc + l.nskip ? j - l.nskip : -1);
 }
+// Where column (j, k) of a tile reads its products at x = 0: a column without any reads
+// the nearest one's, in the lines that its neighbours read (they are multiplied by
+// m = 0, and are NaN exactly when its own would be).
+__host__ __device__ __forceinline__ int prod_column(const ProdLay &l, int j, int k) {
+    const int r = prod_row(l, j);
+    return (r >= 0 ? r : l.jc) * l.kp + (k < l.kc ? k : l.kc - 1);
+}
 
 // ---- batched launches over boxes of one shape ----
 // A batch is a set of boxes that share grid, physics and precision but own

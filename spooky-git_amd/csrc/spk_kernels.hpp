@@ -598,8 +598,8 @@ struct FusedConst {
 // start on whole 128-byte lines (a tile list cut at the mask's edges instead,
 // 86 of 129 columns, ran 20% slower: 1449 against 1207 us at 256^3 FP64 stage
 // 2).  A tile with no column in the mask (fx_masked_tile) transforms no
-// product; in the others a column without products reads the (k_y, k_z) = 0
-// column's and multiplies it by m = 0.
+// product; in the others a column without products transforms its neighbour's
+// (prod_column) and multiplies them by m = 0.
 // Tiles without products are cheaper, and they come in runs of rows: an XCD
 // takes every eighth run of 32 tiles (one per CU at a time, neighbours sharing
 // its L2), and the rows past the masked ones come first.
@@ -669,8 +669,7 @@ __device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restric
     const int kk = col - j * c.kg.nzh;
     // the column in the products
     const unsigned pxs = (unsigned)c.pl.xs;
-    const int prow = kk < c.pl.kc ? prod_row(c.pl, j) : -1;
-    const unsigned pcol = prow >= 0 ? (unsigned)(prow * c.pl.kp + kk) : 0u;
+    const unsigned pcol = (unsigned)prod_column(c.pl, j, kk);
     const int p0 = GRP == 0 ? c.oT : (GRP == 1 ? c.oE : c.oQ);
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
