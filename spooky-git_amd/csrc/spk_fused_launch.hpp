@@ -9,34 +9,33 @@
 
 namespace spk {
 
-template <class T, int N, int LY, int EF, bool STRAT = false>
+template <class T, int N, int LY, int EF, int TC, bool STRAT = false>
 static void launch_ly_mode(int mode, dim3 grid, int bs, hipStream_t st, const cpx<T> *P, const cpx<T> *probe, cpx<double> *U,
                            cpx<T> *S, cpx<T> *W, const FusedConst &fc, const cpx<T> *tw, TimeState *ts,
                            const Batch &bt) {
     switch (mode) {
-        case 1: k_fwdx_epilogue<T, N, LY, 1, EF, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
-        case 2: k_fwdx_epilogue<T, N, LY, 2, EF, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
-        default: k_fwdx_epilogue<T, N, LY, 3, EF, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
+        case 1: k_fwdx_epilogue<T, N, LY, 1, EF, TC, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
+        case 2: k_fwdx_epilogue<T, N, LY, 2, EF, TC, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
+        default: k_fwdx_epilogue<T, N, LY, 3, EF, TC, STRAT><<<grid, bs, 0, st>>>(P, probe, U, S, W, fc, tw, ts, bt); break;
     }
 }
 
 // Boussinesq layouts: stratified runs couple the velocity and temperature
 // groups in one block (k_fwdx_epilogue's STRAT instantiation)
-template <class T, int N, int LY, int EF>
+template <class T, int N, int LY, int EF, int TC>
 static int launch_bouss(int mode, dim3 grid, int bs, hipStream_t st, const cpx<T> *P, const cpx<T> *probe, cpx<double> *U, cpx<T> *S,
                         cpx<T> *W, const FusedConst &fc, const cpx<T> *tw, TimeState *ts, const Batch &bt) {
     if (!fc.e.stratification) {
-        launch_ly_mode<T, N, LY, EF>(mode, grid, bs, st, P, probe, U, S, W, fc, tw, ts, bt);
+        launch_ly_mode<T, N, LY, EF, TC>(mode, grid, bs, st, P, probe, U, S, W, fc, tw, ts, bt);
         return SPK_OK;
     }
-    launch_ly_mode<T, N, LY, EF, true>(mode, grid, bs, st, P, probe, U, S, W, fc, tw, ts, bt);
+    launch_ly_mode<T, N, LY, EF, TC, true>(mode, grid, bs, st, P, probe, U, S, W, fc, tw, ts, bt);
     return SPK_OK;
 }
 
-template <class T, int N, int EF>
-static int launch_n(int ly, int mode, hipStream_t st, const void *P, const void *probe, void *U, void *S, void *W,
-                    const FusedConst &fc, const void *tw, TimeState *ts, int ngroups, const Batch &bt, unsigned nbz) {
-    constexpr int TC = fx_tcols(N, EF);
+template <class T, int N, int EF, int TC>
+static int launch_tc(int ly, int mode, hipStream_t st, const void *P, const void *probe, void *U, void *S, void *W,
+                     const FusedConst &fc, const void *tw, TimeState *ts, int ngroups, const Batch &bt, unsigned nbz) {
     const long long ncols = (long long)fc.e.kg.ny * fc.e.kg.nzh;
     dim3 grid((unsigned)((ncols + TC - 1) / TC), ngroups, nbz);
     const int bs = TC * fx_tpl(N, EF);
@@ -46,14 +45,30 @@ static int launch_n(int ly, int mode, hipStream_t st, const void *P, const void 
     cpx<T> *w = (cpx<T> *)W;
     const cpx<T> *t = (const cpx<T> *)tw;
     switch (ly) {
-        case LY_HD: launch_ly_mode<T, N, LY_HD, EF>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt); break;
-        case LY_HD_TH: SPK_TRY((launch_bouss<T, N, LY_HD_TH, EF>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt))); break;
-        case LY_MHD: launch_ly_mode<T, N, LY_MHD, EF>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt); break;
-        case LY_MHD_TH: SPK_TRY((launch_bouss<T, N, LY_MHD_TH, EF>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt))); break;
+        case LY_HD: launch_ly_mode<T, N, LY_HD, EF, TC>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt); break;
+        case LY_HD_TH: SPK_TRY((launch_bouss<T, N, LY_HD_TH, EF, TC>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt))); break;
+        case LY_MHD: launch_ly_mode<T, N, LY_MHD, EF, TC>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt); break;
+        case LY_MHD_TH: SPK_TRY((launch_bouss<T, N, LY_MHD_TH, EF, TC>(mode, grid, bs, st, p, pr, u, s, w, fc, t, ts, bt))); break;
         default: set_error("fused epilogue: layout %d has no FFT products", ly); return SPK_ERR_STATE;
     }
     SPK_LAUNCH_CHECK();
     return SPK_OK;
+}
+
+// One column of 1024 points at 4 per thread fills a 256-thread block.  Where that makes
+// more blocks than CUs, two columns to a block are faster, whose loads are twice as
+// wide (FP32, us per step, one / two: 1024x128x2 HD, 256 blocks, 119 / 132; the same
+// MHD, 512 blocks, 189 / 150).  The rule counts one box's blocks, so that a batch and
+// its boxes launched one by one take the same tiles.
+template <class T, int N, int EF>
+static int launch_n(int ly, int mode, hipStream_t st, const void *P, const void *probe, void *U, void *S, void *W,
+                    const FusedConst &fc, const void *tw, TimeState *ts, int ngroups, const Batch &bt, unsigned nbz) {
+    constexpr int TC = fx_tcols(N, EF);
+    if constexpr (TC == 1) {
+        if ((long long)fc.e.kg.ny * fc.e.kg.nzh * ngroups > 256)
+            return launch_tc<T, N, EF, 2>(ly, mode, st, P, probe, U, S, W, fc, tw, ts, ngroups, bt, nbz);
+    }
+    return launch_tc<T, N, EF, TC>(ly, mode, st, P, probe, U, S, W, fc, tw, ts, ngroups, bt, nbz);
 }
 
 template <class T, int EF>

@@ -1033,8 +1033,8 @@ __device__ __forceinline__ void fx_masked(const cpx<T> *__restrict__ probe, cpx<
 
 // STRAT (Boussinesq layouts with stratification): the temperature group and
 // then the velocity group in the first grid row's blocks, grid y = 1 + MHD
-template <class T, int N, int LY, int MODE, int EF, bool STRAT = false>
-__global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilogue(
+template <class T, int N, int LY, int MODE, int EF, int TC, bool STRAT = false>
+__global__ __launch_bounds__(TC * fx_tpl(N, EF)) void k_fwdx_epilogue(
     const cpx<T> *P, const cpx<T> *__restrict__ probe, cpx<double> *__restrict__ U, cpx<T> *__restrict__ S,
     cpx<T> *__restrict__ W, FusedConst fc, const cpx<T> *__restrict__ tw, TimeState *ts, Batch bt) {
     using L = Layout<LY>;
@@ -1053,7 +1053,6 @@ __global__ __launch_bounds__(fx_tcols(N, EF) * fx_tpl(N, EF)) void k_fwdx_epilog
     if (MODE == 3 && fc.clock && blockIdx.x + blockIdx.y + threadIdx.x == 0) advance_clock(ts, 1, 1, 1, fc.toutput_flow);
     constexpr int E = fx_e(N, EF);
     constexpr int TPL = N / E;
-    constexpr int TC = fx_tcols(N, EF);
     constexpr int LL = lds_len(N);
     constexpr int NT = TC * TPL;
     __shared__ cpx<T> lds[E != N ? TC * LL : 1];
