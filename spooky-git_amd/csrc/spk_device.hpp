@@ -18,6 +18,8 @@
 
 #include <type_traits>
 
+#include "spk_prodlay.hpp"
+
 namespace spk {
 
 template <class T>
@@ -401,36 +403,6 @@ __host__ __device__ constexpr bool line_needs_lds() {
 __host__ __device__ constexpr int zpass_e(int m) { return line_e(m, 16); }
 __host__ __device__ constexpr int zpass_tpl(int m) { return m / zpass_e(m); }
 __host__ __device__ constexpr int zpass_rw(int m) { return zpass_tpl(m) >= 256 ? 1 : 256 / zpass_tpl(m); }
-
-
-// ---- layout of the RHS products between their z pass and the spectral epilogue ----
-// The 2/3 mask zeroes every product mode with k_z or k_y beyond its threshold,
-// whatever k_x is, so the forward transforms make only the columns the mask
-// keeps: the z pass stores the first kc of NZ/2+1 modes of a row, the y pass
-// transforms those columns and stores the rows with |k_y| index <= jc, moved
-// together (mode j > jc sits in row j - nskip).  At 256^3 that is 86 of 129
-// columns and 171 of 256 rows: the forward y pass reads 0.66 and writes 0.44 of
-// the full spectrum and the x pass reads 0.44 of it (8 fields at 256^3 FP64:
-// y pass 409 -> 254 us, x pass 447 -> 193 us; the FP64 step 6.68 -> 5.97 ms,
-// FP32 bulk 3.95 -> 3.79 ms).  Rows have a pitch of kp elements, a multiple of
-// 128 bytes where a row is long enough (at the full row's 129 elements the y
-// pass took 338 us); planes of one x are xs elements apart.
-// Without a mask kc = kp = NZ/2+1 and every row is kept.
-struct ProdLay {
-    int kc, kp, jc, nskip;
-    long long xs;
-};
-// row of mode j in the products after the forward y pass, -1 where it is masked
-__host__ __device__ __forceinline__ int prod_row(const ProdLay &l, int j) {
-    return j <= l.jc ? j : (j > l.jc + l.nskip ? j - l.nskip : -1);
-}
-// Where column (j, k) of a tile reads its products at x = 0: a column without any reads
-// the nearest one's, in the lines that its neighbours read (they are multiplied by
-// m = 0, and are NaN exactly when its own would be).
-__host__ __device__ __forceinline__ int prod_column(const ProdLay &l, int j, int k) {
-    const int r = prod_row(l, j);
-    return (r >= 0 ? r : l.jc) * l.kp + (k < l.kc ? k : l.kc - 1);
-}
 
 // ---- batched launches over boxes of one shape ----
 // A batch is a set of boxes that share grid, physics and precision but own

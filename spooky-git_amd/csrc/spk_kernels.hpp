@@ -669,7 +669,7 @@ __device__ __forceinline__ void fx_group(const cpx<T> *P, cpx<double> *__restric
     const int kk = col - j * c.kg.nzh;
     // the column in the products
     const unsigned pxs = (unsigned)c.pl.xs;
-    const unsigned pcol = (unsigned)prod_column(c.pl, j, kk);
+    const unsigned pcol = (unsigned)prod_column(c.pl, c.kg.nzh, j, kk);
     const int p0 = GRP == 0 ? c.oT : (GRP == 1 ? c.oE : c.oQ);
     const int lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);

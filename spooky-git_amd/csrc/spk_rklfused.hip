@@ -109,7 +109,7 @@ __global__ __launch_bounds__(rklf_tcols(N) * fx_tpl(N, RKLF_E)) void k_fwdx_rkl2
     // the column in the flux products; element offsets inside a field fit 32 bits
     // and are added to wave-uniform bases
     const unsigned ucol = (unsigned)col, unc = (unsigned)ncols, pxs = (unsigned)c.pl.xs;
-    const unsigned pcol = (unsigned)prod_column(c.pl, j, kk);
+    const unsigned pcol = (unsigned)prod_column(c.pl, c.kg.nzh, j, kk);
     cpx<double> *const Uf = U + F;
 
     for (int e = tid; e < N; e += NT) twl[e] = tw[e];
