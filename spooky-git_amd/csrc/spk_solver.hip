@@ -1382,6 +1382,19 @@ int hydro_mhd_advance(spk_solver s) {
 // with 4 or 8 points per thread against the unfused forward x pass + epilogue +
 // next inverse x pass (+ a third of the projection pass).  Zero state, zero
 // products and a zero step keep every buffer at zero.
+//
+// The times are three launches each, and decide only where they differ clearly, so
+// that solvers of one shape mostly choose alike (and then give the same bits): 5 to 10 of
+// 660 shapes (NX 32..1024, four physics, both precisions) chose otherwise in a second
+// process, 28 when the least time decided.  Programs that need the same bits of two
+// solvers set the back end and the tile (spk_solver_set_fused, spk_solver_set_fused_points).
+//   Points per thread: 8 where that leaves a block for most CUs (measured per stage, us,
+//   4 / 8 points: 64^3 MHD FP64 22 / 29 with 66 blocks, 1024x32x32 111 / 97 with 272),
+//   unless the other is 15% faster.
+//   Fused or not: fused unless the separate kernels are 10% faster, because a fused
+//   stage also saves two launches, which these times do not show.  Steps of the 660 shapes
+//   took 0.2% longer than their best form's on average with this margin and less than 6%
+//   at most; without one 0.5% and 14%, with 15% 0.2% and 6%.
 int tune_fused(spk_solver s) {
     s->fused_ef = 4;
     s->fused_ef_auto = 4;
@@ -1411,11 +1424,6 @@ int tune_fused(spk_solver s) {
         SPK_HIP(hipEventElapsedTime(ms, e0, e1));
         return SPK_OK;
     };
-    // The choice is the tile count's unless another one is clearly (15%) faster,
-    // so that solvers of one shape make the same choice and give the same bits:
-    // 8 points per thread where that leaves a block for most CUs (measured per
-    // stage, us, 4 / 8 points: 64^3 MHD FP64 22 / 29 with 66 blocks, 1024x32x32
-    // 111 / 97 with 272).
     const long long tiles8 = ((long long)g.ny * g.nzh + fx_tcols(g.nx, 8) - 1) / fx_tcols(g.nx, 8);
     float t_fx[2] = {0.f, 0.f}, t_unf = 0.f, t_cl = 0.f;
     int rc = SPK_OK;
@@ -1440,7 +1448,7 @@ int tune_fused(spk_solver s) {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     SPK_TRY(rc);
-    s->fused_faster = 0.85f * t_fx[pick] < t_unf + t_cl / 3.0f;
+    s->fused_faster = 0.9f * t_fx[pick] < t_unf + t_cl / 3.0f;
     s->fused_ef_auto = s->fused_ef;
     return SPK_OK;
 }
@@ -2384,7 +2392,7 @@ extern "C" int spk_kernel_timings(spk_solver s, int reps, double *out_ms, int ca
             FusedConst fc;
             memset(&fc, 0, sizeof(fc));
             fc.e = c;
-                    fc.project = 0;
+            fc.project = 0;
             fc.inv = 1;
             fc.scale = 1.0 / ((double)g.nx * g.ny * g.nz);
             const void *tw = (const char *)s->twb.d + (size_t)s->twb.off_x * (s->bulk == SPK_F64 ? 16 : 8);
