@@ -95,14 +95,12 @@ __device__ __forceinline__ float gelu_d(float z) {
 
 __device__ __forceinline__ int wrap(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
-// Halo points in LDS at a pitch of CIN + 8 channels (80 or 48 bytes): the 16
+// Halo points of the hidden activations in LDS at a pitch of 80 bytes: the 16
 // lanes of one 16-byte read cycle, on consecutive points, then fall on disjoint
 // groups of 4 banks (64 banks of 4 bytes), and every tap's address is the lane's
 // base address plus a constant, so the transform needs no per-tap address registers.
-__host__ __device__ constexpr int xpitch(int cin) { return cin + 8; }
-constexpr size_t conv_lds(int cin) {
-    return (size_t)(NTAP * CH * cin + HX * HY * HZ * xpitch(cin)) * sizeof(bf16) + CH * sizeof(float);
-}
+constexpr int XPITCH = CH + 8;
+constexpr size_t CONV_LDS = (size_t)(NTAP * CH * CH + HX * HY * HZ * XPITCH) * sizeof(bf16) + CH * sizeof(float);
 
 constexpr int CONV_T = 512;  // 8 waves, two per SIMD
 
@@ -155,7 +153,7 @@ struct HaloPrefetch {
         for (int k = 0; k < NPF; k++)
             if (t + k * NT < NCH) v[k] = *reinterpret_cast<const bf16x8 *>(X + (size_t)o[k] * 8);
     }
-    __device__ __forceinline__ void stash(bf16 *Xs, int t, int pitch = xpitch(CIN)) const {
+    __device__ __forceinline__ void stash(bf16 *Xs, int t, int pitch) const {
 #pragma unroll
         for (int k = 0; k < NPF; k++) {
             const int i = t + k * NT;
@@ -204,10 +202,10 @@ __device__ __forceinline__ void spread_point(const u32x4 (&raw)[2], bf16x4 (&v)[
     __builtin_memcpy(v, d, 32);
 }
 
-// MODE 0: hidden layer, Y = GELU(conv + b); 1: also Z = conv + b (training);
-// 2: output layer, out[c][p] = conv + b for c < 6 (FP32, channel-major);
+// Hidden layers and the input gradient, 32 -> 32 channels.
+// MODE 0: Y = GELU(conv + b); 1: also Z = conv + b (training);
 // 3: input gradient, Y = conv(dZ, flipped transposed W) * GELU'(Zp)
-
+//
 // What bounds it: per brick (512 points) the MFMAs, the LDS reads of their
 // operands and the activation's VALU work are of one size, and a wave does them
 // one after the other.  So the two waves of a SIMD take turns: waves 0-3 compute
@@ -219,16 +217,15 @@ __device__ __forceinline__ void spread_point(const u32x4 (&raw)[2], bf16x4 (&v)[
 // stores of a point, 128^3, 32 -> 32 channels: 165 -> 134 us, with the stored Z
 // 180 -> 143, input gradient 190 -> 148.  Inputs in flight and out alone (no matrix
 // work, no activation) take 77 us of that, the MFMAs 46.
-template <int CIN, int MODE>
+template <int MODE>
 __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, const bf16 *__restrict__ W,
                                                  const float *__restrict__ bias, bf16 *__restrict__ Y,
                                                  bf16 *__restrict__ Z, const bf16 *__restrict__ Zp, int n) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    bf16 *Ws = reinterpret_cast<bf16 *>(smem);  // [27][32][CIN], chunk-swizzled by co
-    bf16 *Xs = Ws + NTAP * CH * CIN;            // [HX*HY*HZ][xpitch(CIN)]
-    float *Bs = reinterpret_cast<float *>(Xs + HX * HY * HZ * xpitch(CIN));  // [32]
-    constexpr int NQ = CIN / 8, NKC = CIN / 16, NG = 9 * NKC;
-    static_assert(MODE == 0 || MODE == 1 || MODE == 3, "hidden layers and the input gradient");
+    bf16 *Ws = reinterpret_cast<bf16 *>(smem);  // [27][32][32], chunk-swizzled by co
+    bf16 *Xs = Ws + NTAP * CH * CH;             // [HX*HY*HZ][XPITCH]
+    float *Bs = reinterpret_cast<float *>(Xs + HX * HY * HZ * XPITCH);  // [32]
+    constexpr int NQ = CH / 8, NKC = CH / 16, NG = 9 * NKC;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int xw = w & 3, four = w >> 2;
@@ -236,8 +233,8 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
 
     for (int i = tid; i < NTAP * CH * NQ; i += CONV_T) {
         const int q = i % NQ, row = i / NQ;
-        const bf16x8 v = *reinterpret_cast<const bf16x8 *>(W + (size_t)row * CIN + 8 * q);
-        *reinterpret_cast<bf16x8 *>(Ws + row * CIN + 8 * swz(q, row & 31)) = v;
+        const bf16x8 v = *reinterpret_cast<const bf16x8 *>(W + (size_t)row * CH + 8 * q);
+        *reinterpret_cast<bf16x8 *>(Ws + row * CH + 8 * swz(q, row & 31)) = v;
     }
     Bricks br(n);
     if (MODE != 3 && tid < CH) Bs[tid] = bias[tid];
@@ -285,12 +282,12 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
 #pragma unroll
             for (int dy = 0; dy < 3; dy++) {
                 const int t = 9 * (dx + 1) + 3 * dy + dz + 1;
-                a[g & 1][dy] = *reinterpret_cast<const bf16x8 *>(Ws + (t * CH + li) * CIN + 8 * swz(q, li));
+                a[g & 1][dy] = *reinterpret_cast<const bf16x8 *>(Ws + (t * CH + li) * CH + 8 * swz(q, li));
             }
 #pragma unroll
             for (int yy = 0; yy < 6; yy++) {
                 const int hp = ((xw + 1 + dx) * HY + yy) * HZ + li + 1 + dz;
-                x[g & 1][yy] = *reinterpret_cast<const bf16x8 *>(Xs + hp * xpitch(CIN) + 8 * q);
+                x[g & 1][yy] = *reinterpret_cast<const bf16x8 *>(Xs + hp * XPITCH + 8 * q);
             }
         };
         operands(0);
@@ -307,12 +304,12 @@ __global__ __launch_bounds__(CONV_T) void k_conv(const bf16 *__restrict__ X, con
         }
     };
 
-    HaloPrefetch<CIN, CONV_T> hf(n, tid);
+    HaloPrefetch<CH, CONV_T> hf(n, tid);
     if (br.live()) hf.fetch(X, br, br.k, tid);
     int turn = 0, last = -1;
     for (; br.live(); br.k += br.step, turn ^= 1) {
         __syncthreads();
-        hf.stash(Xs, tid);
+        hf.stash(Xs, tid, XPITCH);
         __syncthreads();
         // the next brick's loads are in flight during this brick's matrix work (the
         // scheduling barrier keeps them ahead of it)
@@ -414,7 +411,7 @@ __global__ void k_pack_in(const float *__restrict__ W, bf16 *__restrict__ Wi) {
 // one instruction per tap and 16-point tile (the 6 stresses in rows 0..5), half
 // the work of a 32-row tile.  out[c][p] = D + b for c < 6.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-constexpr size_t OUT_LDS = (size_t)(NTAP * 16 * CH + HX * HY * HZ * xpitch(CH)) * sizeof(bf16);
+constexpr size_t OUT_LDS = (size_t)(NTAP * 16 * CH + HX * HY * HZ * XPITCH) * sizeof(bf16);
 
 // T = float: out[6][P], for the loss; T = double: the stresses themselves, times
 // their scales, in the padded real layout [6][n][n][n + 2] (pads 0), so that no
@@ -428,7 +425,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
                                                      OutScale sc) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     bf16 *Ws = reinterpret_cast<bf16 *>(smem);  // [27][16][32], chunk-swizzled by co
-    bf16 *Xs = Ws + NTAP * 16 * CH;             // [HX*HY*HZ][xpitch(32)]
+    bf16 *Xs = Ws + NTAP * 16 * CH;             // [HX*HY*HZ][XPITCH]
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int l16 = lane & 15, q = lane >> 4;   // 16x16x32: lane holds row/column l16, K chunk q
     const int xw = w & 3, yg = 2 * (w >> 2);
@@ -447,7 +444,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
         int x0, y0, z0;
         br.origin(br.k, x0, y0, z0);
         __syncthreads();
-        hf.stash(Xs, tid);
+        hf.stash(Xs, tid, XPITCH);
         __syncthreads();
         if (br.more()) hf.fetch(X, br, br.k + br.step, tid);
         __builtin_amdgcn_sched_barrier(0);
@@ -473,7 +470,7 @@ __global__ __launch_bounds__(CONV_T) void k_conv_out(const bf16 *__restrict__ X,
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const int hp = ((xw + 1 + dx) * HY + yg + yy) * HZ + 16 * h + l16 + 1 + dz;
-                    x[yy][h] = *reinterpret_cast<const bf16x8 *>(Xs + hp * xpitch(CH) + 8 * q);
+                    x[yy][h] = *reinterpret_cast<const bf16x8 *>(Xs + hp * XPITCH + 8 * q);
                 }
 #pragma unroll
             for (int dy = 0; dy < 3; dy++)
@@ -912,11 +909,11 @@ void closure_free(spk_closure c) {
 int set_lds_attributes() {
     static bool done = false;
     if (done) return SPK_OK;
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CONV_LDS));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CONV_LDS));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv_out<float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OUT_LDS));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv_out<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)OUT_LDS));
-    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<32, 3>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)conv_lds(32)));
+    SPK_HIP(hipFuncSetAttribute((const void *)k_conv<3>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)CONV_LDS));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv_dw<16>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dw_lds(16)));
     SPK_HIP(hipFuncSetAttribute((const void *)k_conv_dw<32>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)dw_lds(32)));
     done = true;
@@ -957,12 +954,12 @@ int forward(spk_closure c, const void *u, double *tau) {
     for (int l = 0; l < 4; l++) b[l] = c->prm + param_offset(l) + w_count(l);
     if (train) {
         k_conv_in<1><<<gin, 256, 0, st>>>(c->xin4, c->Wb[0], b[0], c->A[0], c->Z[0], c->n);
-        k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], c->Z[1], nullptr, c->n);
-        k_conv<32, 1><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], c->Z[2], nullptr, c->n);
+        k_conv<1><<<g, CONV_T, CONV_LDS, st>>>(c->A[0], c->Wb[1], b[1], c->A[1], c->Z[1], nullptr, c->n);
+        k_conv<1><<<g, CONV_T, CONV_LDS, st>>>(c->A[1], c->Wb[2], b[2], c->A[2], c->Z[2], nullptr, c->n);
     } else {
         k_conv_in<0><<<gin, 256, 0, st>>>(c->xin4, c->Wb[0], b[0], c->A[0], nullptr, c->n);
-        k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[0], c->Wb[1], b[1], c->A[1], nullptr, nullptr, c->n);
-        k_conv<32, 0><<<g, CONV_T, conv_lds(32), st>>>(c->A[1], c->Wb[2], b[2], c->A[2], nullptr, nullptr, c->n);
+        k_conv<0><<<g, CONV_T, CONV_LDS, st>>>(c->A[0], c->Wb[1], b[1], c->A[1], nullptr, nullptr, c->n);
+        k_conv<0><<<g, CONV_T, CONV_LDS, st>>>(c->A[1], c->Wb[2], b[2], c->A[2], nullptr, nullptr, c->n);
     }
     if (train) k_conv_out<float><<<g, CONV_T, OUT_LDS, st>>>(c->A[2], c->Wb[3], b[3], c->out, c->n, out_scale_of(c));
     else k_conv_out<double><<<g, CONV_T, OUT_LDS, st>>>(c->A[2], c->Wb[3], b[3], tau, c->n, out_scale_of(c));
@@ -1075,11 +1072,11 @@ extern "C" int spk_closure_grads(spk_closure c, const void *u, const void *tau_t
     const unsigned g = conv_grid(c);
     // layer 4, then back through layers 3, 2, 1
     SPK_TRY(layer_grads(c, 3, c->A[2], c->dzA));
-    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzA, c->WT[3], nullptr, c->dzB, nullptr, c->Z[2], c->n);
+    k_conv<3><<<g, CONV_T, CONV_LDS, st>>>(c->dzA, c->WT[3], nullptr, c->dzB, nullptr, c->Z[2], c->n);
     SPK_TRY(layer_grads(c, 2, c->A[1], c->dzB));
-    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzB, c->WT[2], nullptr, c->dzA, nullptr, c->Z[1], c->n);
+    k_conv<3><<<g, CONV_T, CONV_LDS, st>>>(c->dzB, c->WT[2], nullptr, c->dzA, nullptr, c->Z[1], c->n);
     SPK_TRY(layer_grads(c, 1, c->A[0], c->dzA));
-    k_conv<32, 3><<<g, CONV_T, conv_lds(32), st>>>(c->dzA, c->WT[1], nullptr, c->dzB, nullptr, c->Z[0], c->n);
+    k_conv<3><<<g, CONV_T, CONV_LDS, st>>>(c->dzA, c->WT[1], nullptr, c->dzB, nullptr, c->Z[0], c->n);
     SPK_TRY(layer_grads(c, 0, c->xin, c->dzB));
     SPK_LAUNCH_CHECK();
     if (loss) {
