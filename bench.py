@@ -159,12 +159,18 @@ KERNEL_NAMES = {
 }
 
 
+def kept_shares(ny, nz):
+    """Shares of a product's modes that the 2/3 mask (|k| <= 2/3 (n/2 - 1)) keeps
+    after the z pass and after the y pass."""
+    fz = (2 * (nz // 2 - 1) // 3 + 1) / (nz // 2 + 1)
+    return fz, fz * (2 * (2 * (ny // 2 - 1) // 3) + 1) / ny
+
+
 def kernel_table(spk, ctx, state, n, prec, fused, reps=10):
     """Live per-kernel average launch time (HIP events, spk_kernel_timings) and
     algorithmic HBM bytes per launch for the MHD step (6 state fields, 8 products);
     fused: the step runs the fused forward-x/epilogue kernel (autotune's choice).
-    The products cross HBM as the modes that the 2/3 mask keeps: kc of the n/2+1
-    columns after the z pass, and the rows |k_y| < kc of those after the y pass."""
+    The products cross HBM as the modes that the 2/3 mask keeps (kept_shares)."""
     sol = spk.Solver(ctx, prec, **mhd_params(n))
     sol.set_fields(state)
     sol.main_loop(1)
@@ -173,9 +179,7 @@ def kernel_table(spk, ctx, state, n, prec, fused, reps=10):
     s64 = n * n * (n // 2 + 1) * 16
     sb = s64 if prec == "f64" else s64 // 2
     nin, nout, nf = 6, 8, 6
-    kc = n // 3 + 1
-    fz = kc / (n // 2 + 1)  # share of a product's modes after the z pass
-    fzy = fz * (2 * kc - 1) / n  # and after the y pass
+    fz, fzy = kept_shares(n, n)
     algo = {"inv_x": nin * (s64 + sb), "inv_y": nin * 2 * sb, "zmid": (nin + nout * fz) * sb,
             "fwd_y": nout * (fz + fzy) * sb, "fwd_x": nout * 2 * fzy * sb,
             "epilogue": nout * fzy * sb + 4 * nf * s64, "clean_div": 2 * nf * s64,
@@ -454,20 +458,23 @@ def box_state(ini, p, seed):
 
 
 def ensemble_bytes(p, bulk_bytes):
-    """Algorithmic HBM bytes of one main-loop step of a box, counted as for the
-    256^3 step: every 3D transform one sweep of its fields (2 S_bulk per field,
-    read + write) and the FP64 RK3 state traffic (U read/write, increment
-    register) of the fused back end; RKL2 stages as 6 transforms + 6 S_64 of
-    state traffic + 3 S_bulk of real-space B per stage (taken from the box's own
-    stage count)."""
+    """Algorithmic HBM bytes of one main-loop step of a box: every 3D transform
+    one sweep of its fields (2 S_bulk per field, read + write; products of the
+    share f of the modes that the 2/3 mask keeps), and the RK3 state traffic of
+    the fused back end: U read in every stage, written in stage 3 and, of the kept
+    modes, in stage 2; of those also the increment register (bulk precision) written in
+    stages 1 and 2 and read in stages 2 and 3.  RKL2 stages: 3 transforms of the
+    gradient, 3 of the flux's kept modes, 6 f S_64 of state traffic, 3 S_bulk of
+    real-space B (times the box's own stage count)."""
     nzh = p["nz"] // 2 + 1
     ntc = p["nx"] * p["ny"] * nzh
     s64, sb = 16 * ntc, bulk_bytes * ntc
     nf = 3 + (3 if p.get("mhd") else 0) + (1 if p.get("boussinesq") else 0)
     nin = nf
     nout = 5 + (3 if p.get("mhd") else 0) + (3 if p.get("boussinesq") else 0)
-    transforms = 3 * (nin + nout)
-    return 2 * transforms * sb + 7 * nf * s64, 6 * 2 * sb + 6 * s64 + 3 * sb
+    f = kept_shares(p["ny"], p["nz"])[1]
+    return (6 * (nin + nout * f) * sb + nf * ((4 + f) * s64 + 4 * f * sb),
+            (6 + 6 * f) * sb + 6 * f * s64 + 3 * sb)
 
 
 def ensemble_leg(spk, ini, ctx, steps, acc_steps=10, split=-1, group="all"):

@@ -596,7 +596,7 @@ struct FusedConst {
 // Column tiles of the fused kernel: tile T holds the TC columns from T TC on of
 // the flattened (k_y, k_z) index, so that its accesses to the state and to W
 // start on whole 128-byte lines (a tile list cut at the mask's edges instead,
-// 86 of 129 columns, ran 20% slower: 1449 against 1207 us at 256^3 FP64 stage
+// 85 of 129 columns, ran 20% slower: 1449 against 1207 us at 256^3 FP64 stage
 // 2).  A tile with no column in the mask (fx_masked_tile) transforms no
 // product; in the others a column without products transforms its neighbour's
 // (prod_column) and multiplies them by m = 0.

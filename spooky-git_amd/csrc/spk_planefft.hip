@@ -53,7 +53,7 @@ struct PlaneShape {
     static constexpr int TPLY = NY / EY, TC = PF_T / TPLY;
     static constexpr int ROWS = NY + (RW > NY ? 1 : 0);  // a spare row for row groups past the plane
     static constexpr size_t bytes = (size_t)ROWS * LL * sizeof(cpx<T>);
-    static constexpr bool fits = bytes <= PF_LDS && TPLZ <= 64 && NY >= 8;
+    static constexpr bool fits = bytes <= PF_LDS && TPLZ <= 64;
 };
 
 template <class T, int NY, int NZ, int DIR>

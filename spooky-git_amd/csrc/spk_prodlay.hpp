@@ -8,13 +8,12 @@ namespace spk {
 // whatever k_x is, so the forward transforms make only the columns the mask
 // keeps: the z pass stores the first kc of NZ/2+1 modes of a row, the y pass
 // transforms those columns and stores the rows with |k_y| index <= jc, moved
-// together (mode j > jc sits in row j - nskip).  At 256^3 that is 86 of 129
-// columns and 171 of 256 rows: the forward y pass reads 0.66 and writes 0.44 of
-// the full spectrum and the x pass reads 0.44 of it (8 fields at 256^3 FP64:
-// y pass 409 -> 254 us, x pass 447 -> 193 us; the FP64 step 6.68 -> 5.97 ms,
-// FP32 bulk 3.95 -> 3.79 ms).  Rows have a pitch of kp elements, a multiple of
-// 128 bytes where a row is long enough (at the full row's 129 elements the y
-// pass took 338 us); planes of one x are xs elements apart.
+// together (mode j > jc sits in row j - nskip).  At 256^3 that is 85 of 129
+// columns and 169 of 256 rows: the forward y pass reads 0.66 and writes 0.43 of
+// the full spectrum and the x pass reads 0.43 of it (8 fields at 256^3 FP64:
+// y pass 409 -> 254 us, x pass 447 -> 193 us).  Rows have a pitch of kp elements
+// (88 there), a multiple of 128 bytes where a row is long enough (at the full row's
+// 129 elements the y pass took 338 us); planes of one x are xs elements apart.
 // Without a mask kc = kp = NZ/2+1 and every row is kept.
 struct ProdLay {
     int kc, kp, jc, nskip;

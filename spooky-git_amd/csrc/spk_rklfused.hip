@@ -27,7 +27,7 @@
 // tile without products therefore does nothing, and its A and B stay those of
 // stage 1: the y pass writes the gradient beside them, not over them.  Per
 // stage at 256^3 this moves 20 field sweeps instead of 29 (y pass 5, z kernel 9
-// -> 8, forward y 5 -> 2.9, this kernel 10 -> 4.8).
+// -> 8, forward y 5 -> 2.9, this kernel 10 -> 4.4).
 #include "spk_internal.hpp"
 #include "spk_kernels.hpp"
 
